@@ -39,6 +39,8 @@
 // Long sequences are bound by exp + MFMA issue: a wavefront then takes two
 // query tiles at once, sharing each K and V^T operand read between them.
 
+#include <algorithm>
+
 #include "kernels.h"
 
 namespace bbh {
@@ -366,31 +368,73 @@ hipError_t attention_packed(const f16* qkv, const PackedSentence* sents, int n, 
 namespace {
 
 // ---- unfused pieces with the reference's launcher shapes -------------------
+// The operands may sit at any element address (only scores' qkv is checked
+// for 16 bytes), so these kernels move 16 and 8 bytes at a time through types
+// that promise 2-byte alignment: gfx950 takes such global accesses at any
+// address, in one instruction.
+typedef f16x8 f16x8_any __attribute__((aligned(2)));
+typedef f16x4 f16x4_any __attribute__((aligned(2)));
+typedef int32_t i32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
 // scores[z, i, j] = scale * sum_d Q[b, i, d] K[b, j, d], z = b*heads + h
-// (src/kernels/attention.cu:17-60), fp32 accumulate, fp16 store.
+// (src/kernels/attention.cu:17-60), fp32 accumulate, fp16 store.  seq % 16 == 0.
+//
+// Bound by writing the scores.  A wavefront makes 32 queries x 64 keys (two
+// 32x32 MFMA tiles, two k-steps each, operands straight from global memory)
+// and stores them through its own LDS tile as 128-byte row runs; a workgroup
+// of four covers 128 queries, so its K rows are fetched once into the L1.
+// One value per thread (two 64-byte row reads for each 2-byte store) took
+// 58.9 us at batch 32 x seq 128, against 9.3 us here (12.6 MB out).
+constexpr int kScoreKeys = 64, kScoreLd = kScoreKeys + 8;
 __global__ __launch_bounds__(256) void scores_kernel(const f16* __restrict__ qkv,
                                                      f16* __restrict__ scores, int heads,
                                                      int seq, int ld, int q_off, int k_off_,
                                                      float scale) {
+  __shared__ __align__(16) f16 stage[4][32 * kScoreLd];
+  const int kblocks = (seq + kScoreKeys - 1) / kScoreKeys;
   const int z = blockIdx.y, b = z / heads, h = z % heads;
-  const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= (size_t)seq * seq) return;
-  const int i = idx / seq, j = idx % seq;
-  const f16* qr = qkv + ((size_t)b * seq + i) * ld + q_off + h * kHeadDim;
-  const f16* kr = qkv + ((size_t)b * seq + j) * ld + k_off_ + h * kHeadDim;
-  float acc = 0.f;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r32 = lane & 31, kh = lane >> 5;
+  const int q0 = ((int)(blockIdx.x / kblocks) * 4 + wave) * 32;
+  const int k0 = (int)(blockIdx.x % kblocks) * kScoreKeys;
+  if (q0 >= seq) return;  // no barrier follows: each wavefront keeps to its own LDS tile
+  const f16* base = qkv + (size_t)b * seq * ld + h * kHeadDim + 8 * kh;
+  // Rows past the sequence read its last row; what they give is not stored.
+  const f16* qr = base + (size_t)min(q0 + r32, seq - 1) * ld + q_off;
+  const f16x8 qa = *reinterpret_cast<const f16x8_any*>(qr);
+  const f16x8 qb = *reinterpret_cast<const f16x8_any*>(qr + 16);
+  f16x8 ka[2], kb[2];
 #pragma unroll
-  for (int d = 0; d < kHeadDim; d += 8) {
-    const f16x8 a = *reinterpret_cast<const f16x8*>(qr + d);
-    const f16x8 c = *reinterpret_cast<const f16x8*>(kr + d);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) acc += (float)a[e] * (float)c[e];
+  for (int t = 0; t < 2; ++t) {
+    const f16* kr = base + (size_t)min(k0 + 32 * t + r32, seq - 1) * ld + k_off_;
+    ka[t] = *reinterpret_cast<const f16x8_any*>(kr);
+    kb[t] = *reinterpret_cast<const f16x8_any*>(kr + 16);
   }
-  scores[(size_t)z * seq * seq + idx] = (f16)(acc * scale);
+  f16* st = stage[wave];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    f32x16 s = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    s = mfma32(ka[t], qa, s);
+    s = mfma32(kb[t], qb, s);  // s[i]: query r32, key k0 + 32t + 8*(i/4) + 4*kh + i%4
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      f16x4 w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[e] = (f16)(s[4 * j + e] * scale);
+      *reinterpret_cast<f16x4*>(st + r32 * kScoreLd + 32 * t + 8 * j + 4 * kh) = w;
+    }
+  }
+  f16* dst = scores + ((size_t)z * seq + q0) * seq + k0;
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    const int row = 8 * p + (lane >> 3), c = (lane & 7) * 8;
+    const f16x8 w = *reinterpret_cast<const f16x8*>(st + row * kScoreLd + c);
+    if (q0 + row < seq && k0 + c < seq)
+      *reinterpret_cast<f16x8_any*>(dst + (size_t)row * seq + c) = w;
+  }
 }
 
-// Row softmax in place, one wavefront per row (src/kernels/softmax.cu:26-63).
+// Row softmax in place, one wavefront per row (src/kernels/softmax.cu:26-63):
+// any N.
 __global__ __launch_bounds__(256) void softmax_kernel(f16* x, int M, int N,
                                                       const int32_t* __restrict__ mask,
                                                       int mask_stride) {
@@ -412,11 +456,71 @@ __global__ __launch_bounds__(256) void softmax_kernel(f16* x, int M, int N,
     r[i] = (mr && mr[i] == 0) ? (f16)0.f : (f16)(__expf((float)r[i] - m) * inv);
 }
 
-// merged[b*seq+i, h*32+d] = sum_j P[z, i, j] V[b, j, d] (attention.cu:65-93).
-__global__ __launch_bounds__(256) void context_kernel(const f16* __restrict__ probs,
-                                                      const f16* __restrict__ qkv,
-                                                      f16* __restrict__ merged, int heads,
-                                                      int seq, int ld, int v_off) {
+// The same for N % 8 == 0 up to 512: LPR lanes hold a row, eight values each
+// (the smallest power of two that covers it), so a wavefront takes 64 / LPR
+// rows and reads and writes each value once, 16 bytes a lane.  Bound by the
+// bytes: 49152 rows of 128 took 23.9 us in three 2-byte passes a row, against
+// 8.5 us here.
+template <int LPR, class F>
+__device__ __forceinline__ float lanes_reduce(float v, F f) {
+  if constexpr (LPR > 32) v = xor_op<32>(v, f);
+  if constexpr (LPR > 16) v = xor_op<16>(v, f);
+  if constexpr (LPR > 8) v = xor_op<8>(v, f);
+  if constexpr (LPR > 4) v = xor_op<4>(v, f);
+  if constexpr (LPR > 2) v = xor_op<2>(v, f);
+  if constexpr (LPR > 1) v = xor_op<1>(v, f);
+  return v;
+}
+template <int LPR>
+__global__ __launch_bounds__(256) void softmax8_kernel(f16* x, int M, int N,
+                                                       const int32_t* __restrict__ mask,
+                                                       int mask_stride) {
+  const int lane = threadIdx.x & 63, c = (lane % LPR) * 8;
+  const int row = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 / LPR) + lane / LPR;
+  const bool in = row < M && c < N;  // the other lanes still take part in the reductions
+  f16* r = x + (size_t)row * N + c;
+  f16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
+  uint32_t on = 0;  // bit e: value e counts
+  if (in) {
+    v = *reinterpret_cast<const f16x8_any*>(r);
+    on = 0xff;
+    if (mask) {
+      const int32_t* mr = mask + (mask_stride > 0 ? (size_t)(row / mask_stride) * N : 0) + c;
+      const i32x4_any m0 = *reinterpret_cast<const i32x4_any*>(mr);
+      const i32x4_any m1 = *reinterpret_cast<const i32x4_any*>(mr + 4);
+      on = 0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) on |= (m0[e] != 0 ? 1u << e : 0u) | (m1[e] != 0 ? 16u << e : 0u);
+    }
+  }
+  float m = -INFINITY;
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    if (on & (1u << e)) m = fmaxf(m, (float)v[e]);
+  m = lanes_reduce<LPR>(m, MaxOp{});
+  float p[8], s = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    p[e] = 0.f;
+    if (on & (1u << e)) {
+      p[e] = __expf((float)v[e] - m);
+      s += p[e];
+    }
+  }
+  s = lanes_reduce<LPR>(s, AddOp{});
+  const float inv = s > 0.f ? 1.0f / s : 0.f;
+  if (!in) return;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = (on & (1u << e)) ? (f16)(p[e] * inv) : (f16)0.f;
+  *reinterpret_cast<f16x8_any*>(r) = v;
+}
+
+// merged[b*seq+i, h*32+d] = sum_j P[z, i, j] V[b, j, d] (attention.cu:65-93):
+// any seq, one value per thread.
+__global__ __launch_bounds__(256) void context1_kernel(const f16* __restrict__ probs,
+                                                       const f16* __restrict__ qkv,
+                                                       f16* __restrict__ merged, int heads,
+                                                       int seq, int ld, int v_off) {
   const int z = blockIdx.y, b = z / heads, h = z % heads;
   const int idx = blockIdx.x * 256 + threadIdx.x;
   if (idx >= seq * kHeadDim) return;
@@ -428,30 +532,132 @@ __global__ __launch_bounds__(256) void context_kernel(const f16* __restrict__ pr
   merged[((size_t)b * seq + i) * heads * kHeadDim + h * kHeadDim + d] = (f16)acc;
 }
 
+// The same for seq % 16 == 0 on the matrix cores: a wavefront makes 32
+// queries x 32 dims as O^T = V^T . P^T.  The probabilities are the B operand
+// as they lie (a lane's eight keys are contiguous); V is staged transposed
+// in LDS, kCtxKeys keys at a time, for the workgroup's NW query tiles.
+// Bound by reading the probabilities: batch 32 x seq 128 took 107 us with one
+// value per thread (a chain of seq dependent adds), against 6.5 us here.
+constexpr int kCtxKeys = 512;
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void context_kernel(const f16* __restrict__ probs,
+                                                          const f16* __restrict__ qkv,
+                                                          f16* __restrict__ merged, int heads,
+                                                          int seq, int ld, int v_off) {
+  HIP_DYNAMIC_SHARED(f16, Vt);  // [32][min(seq, kCtxKeys) + 8]
+  const int vld = min(seq, kCtxKeys) + 8;
+  const int z = blockIdx.y, b = z / heads, h = z % heads;
+  const int tid = threadIdx.x, lane = tid & 63, r32 = lane & 31, kh = lane >> 5;
+  const int q = ((int)blockIdx.x * NW + (tid >> 6)) * 32 + r32;
+  const f16* pr = probs + ((size_t)z * seq + min(q, seq - 1)) * seq + 8 * kh;
+  const f16* vb = qkv + (size_t)b * seq * ld + v_off + h * kHeadDim;
+  f32x16 o = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  // The probabilities of up to 128 keys are loaded together (eight k-steps;
+  // seq is uniform, so a shorter end only skips steps), the first ones before
+  // V is staged.
+  f16x8 p[8];
+  auto load_p = [&](int k) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (k + 16 * u < seq) p[u] = *reinterpret_cast<const f16x8_any*>(pr + k + 16 * u);
+  };
+  load_p(0);
+  for (int k0 = 0; k0 < seq; k0 += kCtxKeys) {
+    const int nk = min(kCtxKeys, seq - k0);
+    if (k0 > 0) __syncthreads();
+    for (int i = tid; i < nk * 2; i += 64 * NW) {  // a 4-key x 4-dim block per thread
+      const int dq = i & 7, kq = i >> 3;
+      f16x4 r[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        r[e] = *reinterpret_cast<const f16x4_any*>(vb + (size_t)(k0 + 4 * kq + e) * ld + 4 * dq);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const f16x4 col = {r[0][e], r[1][e], r[2][e], r[3][e]};
+        *reinterpret_cast<f16x4*>(Vt + (4 * dq + e) * vld + 4 * kq) = col;
+      }
+    }
+    __syncthreads();
+    const f16* vt = Vt + r32 * vld + 8 * kh;
+    for (int k = 0; k < nk; k += 128) {
+      if (k0 + k > 0) load_p(k0 + k);
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (k + 16 * u < nk)  // o[i] = O[q][8*(i/4) + 4*kh + i%4]
+          o = mfma32(*reinterpret_cast<const f16x8*>(vt + k + 16 * u), p[u], o);
+    }
+  }
+  if (q >= seq) return;
+  f16* dst = merged + (((size_t)b * seq + q) * heads + h) * kHeadDim + 4 * kh;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    f16x4 w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w[e] = (f16)o[4 * j + e];
+    *reinterpret_cast<f16x4_any*>(dst + 8 * j) = w;
+  }
+}
+
+template <int NW>
+void launch_context(const f16* probs, const f16* qkv, f16* merged, int batch, int heads, int seq,
+                    int ld, int v_off, hipStream_t s) {
+  const int tiles = (seq + 31) / 32;
+  const size_t lds = (size_t)kHeadDim * (std::min(seq, kCtxKeys) + 8) * sizeof(f16);
+  hipLaunchKernelGGL(context_kernel<NW>, dim3((tiles + NW - 1) / NW, batch * heads), dim3(64 * NW),
+                     lds, s, probs, qkv, merged, heads, seq, ld, v_off);
+}
+
 }  // namespace
 
 
 hipError_t attention_scores(const f16* qkv, f16* scores, int batch, int heads, int seq,
                             int qkv_stride, int q_off, int k_off_, float scale,
                             hipStream_t s) {
-  dim3 grid((unsigned)(((size_t)seq * seq + 255) / 256), batch * heads);
-  hipLaunchKernelGGL(scores_kernel, grid, dim3(256), 0, s, qkv, scores, heads, seq,
-                     qkv_stride, q_off, k_off_, scale);
+  const unsigned qblocks = (seq + 127) / 128, kblocks = (seq + kScoreKeys - 1) / kScoreKeys;
+  hipLaunchKernelGGL(scores_kernel, dim3(qblocks * kblocks, batch * heads), dim3(256), 0, s, qkv,
+                     scores, heads, seq, qkv_stride, q_off, k_off_, scale);
   return hipGetLastError();
 }
 
+// A row of up to 512 values in multiples of eight stays in the registers of
+// up to 64 lanes; other rows take three passes over memory.
 hipError_t softmax_rows(f16* x, int M, int N, const int32_t* mask, int mask_stride,
                         hipStream_t s) {
-  hipLaunchKernelGGL(softmax_kernel, dim3((M + 3) / 4), dim3(256), 0, s, x, M, N, mask,
-                     mask_stride);
+#define BBH_SOFTMAX8(LPR)                                                                   \
+  hipLaunchKernelGGL(softmax8_kernel<LPR>, dim3((M + 256 / LPR - 1) / (256 / LPR)), dim3(256), 0, \
+                     s, x, M, N, mask, mask_stride)
+  if (N % 8 != 0 || N > 512)
+    hipLaunchKernelGGL(softmax_kernel, dim3((M + 3) / 4), dim3(256), 0, s, x, M, N, mask,
+                       mask_stride);
+  else if (N <= 16)
+    BBH_SOFTMAX8(2);
+  else if (N <= 32)
+    BBH_SOFTMAX8(4);
+  else if (N <= 64)
+    BBH_SOFTMAX8(8);
+  else if (N <= 128)
+    BBH_SOFTMAX8(16);
+  else if (N <= 256)
+    BBH_SOFTMAX8(32);
+  else
+    BBH_SOFTMAX8(64);
+#undef BBH_SOFTMAX8
   return hipGetLastError();
 }
 
+// The matrix cores take 16 keys a step, so other lengths go one value a
+// thread.  Up to four query tiles share a workgroup's staged V.
 hipError_t attention_context(const f16* probs, const f16* qkv, f16* merged, int batch,
                              int heads, int seq, int qkv_stride, int v_off, hipStream_t s) {
-  dim3 grid((seq * kHeadDim + 255) / 256, batch * heads);
-  hipLaunchKernelGGL(context_kernel, grid, dim3(256), 0, s, probs, qkv, merged, heads, seq,
-                     qkv_stride, v_off);
+  if (seq % 16 != 0)
+    hipLaunchKernelGGL(context1_kernel, dim3((seq * kHeadDim + 255) / 256, batch * heads),
+                       dim3(256), 0, s, probs, qkv, merged, heads, seq, qkv_stride, v_off);
+  else if (seq <= 32)
+    launch_context<1>(probs, qkv, merged, batch, heads, seq, qkv_stride, v_off, s);
+  else if (seq <= 64)
+    launch_context<2>(probs, qkv, merged, batch, heads, seq, qkv_stride, v_off, s);
+  else
+    launch_context<4>(probs, qkv, merged, batch, heads, seq, qkv_stride, v_off, s);
   return hipGetLastError();
 }
 

@@ -348,6 +348,51 @@ def test_unfused_attention_pieces_match_fused(torch_cuda):
     assert np.abs(_np(fused) - _np(merged)).max() <= TOL
 
 
+@pytest.mark.parametrize("B,S,off", [(1, 16, 0), (3, 48, 1), (2, 80, 0), (2, 128, 3), (1, 144, 0),
+                                     (1, 528, 1), (2, 33, 0), (1, 520, 1), (1, 1040, 0)])
+def test_unfused_attention_pieces_edges(torch_cuda, B, S, off):
+    # Tile edges of the three operators (32 queries, 64 keys, 16-key steps,
+    # 512 staged keys, rows of 2 to 64 lanes and longer), lengths that only the
+    # general kernels take (S % 16), and buffers at odd element addresses.
+    # Each is compared with float64 on its own fp16 input; bounds: fp16
+    # rounding 2^-11 plus the fp32 sums' S * 2^-24 of the absolute sum, both
+    # doubled.
+    torch = torch_cuda
+    from bbh import engine
+
+    rng = np.random.default_rng(S)
+    H, ld, scale = 3, 3 * 96 + 8, 1.0 / np.sqrt(32)
+    qkv = _h(rng, (B * S, ld), 1.5)
+    tq = to_dev(torch, qkv)
+    q, k, v = (qkv[:, o:o + 96].astype(np.float64).reshape(B, S, H, 32).transpose(0, 2, 1, 3)
+               for o in (8, 104, 200))
+    mask = _masks(rng, B, S, "random")
+    mask[-1] = 0  # every key masked: zero probabilities
+    scores = torch.zeros(B * H * S * S + off, dtype=torch.float16, device="cuda")[off:]
+    if S % 16 == 0:
+        engine.launch_attention_scores(tq, scores, B, H, S, 32, ld, 8, 104, scale)
+        want = np.matmul(q, k.transpose(0, 1, 3, 2)) * scale
+        mag = np.matmul(np.abs(q), np.abs(k).transpose(0, 1, 3, 2)) * scale
+        got = _np(scores).reshape(want.shape)
+        assert np.all(np.abs(got - want) <= 2 ** -10 * np.abs(want) + 32 * 2 ** -23 * mag)
+    else:
+        scores += to_dev(torch, _h(rng, (B * H * S * S,), 2.0))
+    x = _np(scores).reshape(B, H, S, S).astype(np.float64)
+    engine.launch_softmax(scores, B * H * S, S, to_dev(torch, mask), H * S)
+    m = mask[:, None, None, :] != 0
+    e = np.where(m, np.exp(x - np.max(np.where(m, x, -1e9), -1, keepdims=True)), 0.0)
+    want = e / np.maximum(e.sum(-1, keepdims=True), 1e-300)
+    probs = _np(scores).reshape(want.shape)
+    assert np.all(np.abs(probs - want) <= (2 ** -10 + S * 2 ** -23) * want + 2 ** -23)
+    out = torch.empty(B * S * H * 32 + off, dtype=torch.float16, device="cuda")[off:]
+    engine.launch_attention_context(scores, tq, out, B, H, S, 32, ld, 200)
+    p = probs.astype(np.float64)
+    want = np.matmul(p, v).transpose(0, 2, 1, 3).reshape(B * S, H * 32)
+    mag = np.matmul(p, np.abs(v)).transpose(0, 2, 1, 3).reshape(B * S, H * 32)
+    got = _np(out).reshape(want.shape)
+    assert np.all(np.abs(got - want) <= 2 ** -10 * np.abs(want) + S * 2 ** -23 * mag + 2 ** -24)
+
+
 def test_softmax_reference_kat(torch_cuda, kats):
     torch = torch_cuda
     from bbh import engine
