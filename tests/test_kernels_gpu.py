@@ -393,6 +393,45 @@ def test_unfused_attention_pieces_edges(torch_cuda, B, S, off):
     assert np.all(np.abs(got - want) <= 2 ** -10 * np.abs(want) + S * 2 ** -23 * mag + 2 ** -24)
 
 
+@pytest.mark.parametrize("B,S,D,off", [(1, 1, 8, 0), (3, 7, 384, 1), (2, 512, 384, 0), (2, 40, 1032, 0),
+                                       (5, 33, 100, 0), (1, 90, 8200, 0), (2, 3, 512, 1)])
+def test_row_operators_edges(torch_cuda, B, S, D, off):
+    # embedding, mean pool and L2 normalise at any width (the vector kernels
+    # take D % 8 == 0, up to 8192 and 512 columns), at odd element addresses,
+    # with an all-masked sentence; NaN in masked rows is not read.  Bounds as
+    # above; the embedding is exact up to its fp16 rounding.
+    torch = torch_cuda
+    from bbh import engine
+
+    rng = np.random.default_rng(D + S)
+    at = lambda a: to_dev(torch, np.concatenate([np.zeros(off, a.dtype), a.ravel()]))[off:]  # noqa: E731
+    word, pos, typ = np.zeros((30522, D), np.float16), _h(rng, (S, D)), _h(rng, (2, D))
+    rows = rng.integers(0, 30522, 64)
+    word[rows] = _h(rng, (64, D))
+    ids = rng.choice(rows, (B, S)).astype(np.int32)
+    types = rng.integers(0, 2, (B, S)).astype(np.int32)
+    out = torch.empty(B * S * D + off, dtype=torch.float16, device="cuda")[off:]
+    engine.launch_embedding(to_dev(torch, ids), to_dev(torch, types), at(word), at(pos), at(typ), out,
+                            S, D, B)
+    f = lambda a: a.astype(np.float32)  # noqa: E731
+    want = ((f(word)[ids] + f(pos)[None]) + f(typ)[types]).astype(np.float16)
+    assert np.array_equal(out.cpu().numpy().reshape(B, S, D), want)
+    h = _h(rng, (B, S, D))
+    mask = _masks(rng, B, S, "random")
+    mask[B - 1] = B == 1
+    h[mask == 0] = np.nan
+    pooled = torch.empty(B * D + off, dtype=torch.float16, device="cuda")[off:]
+    engine.launch_mean_pool(at(h), to_dev(torch, mask), pooled, S, D, B)
+    hz, n = np.where(mask[..., None] != 0, h, 0).astype(np.float64), np.maximum(mask.sum(1), 1)[:, None]
+    want, mag = hz.sum(1) / n, np.abs(hz).sum(1) / n
+    got = _np(pooled).reshape(B, D)
+    assert np.all(np.abs(got - want) <= 2 ** -10 * np.abs(want) + S * 2 ** -23 * mag + 2 ** -24)
+    engine.launch_l2_normalize(pooled, D, B)
+    want = got / np.maximum(np.linalg.norm(got.astype(np.float64), axis=1, keepdims=True), 1e-12)
+    got = _np(pooled).reshape(B, D)
+    assert np.all(np.abs(got - want) <= (2 ** -10 + D * 2 ** -23) * np.abs(want) + 2 ** -24)
+
+
 def test_softmax_reference_kat(torch_cuda, kats):
     torch = torch_cuda
     from bbh import engine
