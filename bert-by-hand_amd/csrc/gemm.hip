@@ -48,15 +48,19 @@ enum Epi { kBias = 0, kGelu = 1, kResidual = 2, kLayerNorm = 3, kFold = 4, kFold
 template <int BM_, int BN_, int WM_, int WN_, int SA_, int PD_ = 0, int SW_ = 2>
 struct Cfg {
   static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, SA = SA_, SW = SW_, BK = 64;
-  // PD_ > 0: register prefetch depth (mainloop_reg); PD_ < 0: the copy-ring
-  // loop with KPB = -PD_ K slices per barrier (mainloop_multi).
+  // PD_ > 0: register prefetch depth (mainloop_reg).  PD_ = -(16 NP + KPB):
+  // one ring of whole slices (mainloop_deep), KPB of them per barrier, copied
+  // by NP wavefronts of their own beside the WM x WN that compute (NP = 0: by
+  // those).
   static constexpr int PD = PD_ > 0 ? PD_ : 0;
-  static constexpr int KPB = PD_ < 0 ? -PD_ : 1;
+  static constexpr int KPB = PD_ < 0 ? -PD_ % 16 : 1, NP = PD_ < 0 ? -PD_ / 16 : 0;
   using L = Slice<64>;
-  static constexpr int NW = WM * WN, THREADS = 64 * NW;  // 4 or 8 wavefronts
+  static constexpr int NW = WM * WN, THREADS = 64 * (NW + NP);
+  static constexpr int NC = NP > 0 ? NP : NW;            // wavefronts that issue the copies
+  static constexpr bool DEEP = PD_ < 0;
   static constexpr int TM = BM / WM, TN = BN / WN;  // wave tile
   static constexpr int FM = TM / 32, FN = TN / 32;  // 32x32 blocks per wave
-  static constexpr int LA = BM / (8 * NW), LW = BN / (8 * NW);  // copies per thread per slice
+  static constexpr int LA = BM / (8 * NC), LW = BN / (8 * NC);  // copies per thread per slice
   static constexpr int A_STAGE = BM * BK, W_STAGE = BN * BK;  // halves per slice
   static constexpr int W_BASE = SA * A_STAGE;                 // W ring follows the A ring
   static constexpr int OUT_LD = BN + 8;                       // padded row of the fp16 output tile
@@ -69,17 +73,16 @@ struct Cfg {
   static constexpr int NPASS = ((size_t)BM * OUT_LD * sizeof(f16) + RED <= kLdsMax) ? 1 : WM;
   static constexpr size_t OUT = (size_t)(BM / NPASS) * OUT_LD * sizeof(f16) + RED;
   static constexpr size_t LDS = RING > OUT ? RING : OUT;
-  static_assert(NW == 4 || NW == 6 || NW == 8, "four, six or eight wavefronts");
+  static_assert(NW + NP <= 16, "wavefronts");
   static_assert(TM % 32 == 0 && TN % 32 == 0, "wave tile is whole 32x32 blocks");
-  static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "load distribution");
+  static_assert(BM % (8 * NC) == 0 && BN % (8 * NC) == 0, "load distribution");
   static_assert(SA >= 2 && SW >= 2, "ring depths");
-  static_assert(KPB == 1 || (PD == 0 && SA == 2 * KPB && SW == 2 * KPB),
-                "KPB slices per barrier: rings of 2 * KPB slices");
+  static_assert(!DEEP || (SA == SW && SA % KPB == 0 && SA >= 2 * KPB), "one ring of whole groups");
   // vmcnt that may stay outstanding when slice kt must have landed: the
   // copies issued after the later of W(kt) and A(kt) (W is issued first in
   // each iteration).
   static constexpr int VM_AHEAD = ((SA < SW ? SA : SW) - 2) * (LA + LW) + (SW < SA ? LA : 0);
-  static_assert(VM_AHEAD < 64, "vmcnt range");
+  static_assert(DEEP || VM_AHEAD < 64, "vmcnt range");
   static_assert(LDS <= kLdsMax, "LDS");
   static_assert(PD == 0 || (BM * 8 % THREADS == 0 && BN * 8 % THREADS == 0), "chunks");
 };
@@ -93,9 +96,14 @@ struct Cfg {
 // resource, the slice's K offset being the instruction's scalar operand.  A
 // K loop so pays no per-lane address arithmetic per copy (on the SIMD issue
 // the MFMAs share: ~65 VALU instructions per wavefront per slice before).
+// NW wavefronts share the copies; `wave` is this one's number among them.
+__device__ __forceinline__ int wave_id() {
+  return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+}
 template <int ROWS, int NW>
-__device__ __forceinline__ void row_offsets(int ld, int valid, uint32_t (&off)[ROWS / (8 * NW)]) {
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+__device__ __forceinline__ void row_offsets(int ld, int valid, uint32_t (&off)[ROWS / (8 * NW)],
+                                            int wave = wave_id()) {
+  const int lane = threadIdx.x & 63;
 #pragma unroll
   for (int j = 0; j < ROWS / (8 * NW); ++j) {
     const int r = (wave * (ROWS / (8 * NW)) + j) * 8 + (lane >> 3);
@@ -107,8 +115,8 @@ __device__ __forceinline__ void row_offsets(int ld, int valid, uint32_t (&off)[R
 // `soff` bytes (wave-uniform).
 template <int ROWS, int NW>
 __device__ __forceinline__ void issue_rows_at(__amdgpu_buffer_rsrc_t src, uint32_t soff,
-                                              const uint32_t (&off)[ROWS / (8 * NW)], f16* buf) {
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+                                              const uint32_t (&off)[ROWS / (8 * NW)], f16* buf,
+                                              int wave = wave_id()) {
 #pragma unroll
   for (int j = 0; j < ROWS / (8 * NW); ++j)
     __builtin_amdgcn_raw_ptr_buffer_load_lds(
@@ -234,17 +242,66 @@ __device__ __forceinline__ void mainloop(const f16* __restrict__ A, const f16* _
   lds_barrier();  // ring free for the epilogue
 }
 
-// The copy-ring K loop with KPB slices per barrier: rings of 2 * KPB slices
-// for A and W.  Iteration k0 waits for slices k0 .. k0+KPB-1 (the copies
-// issued one iteration earlier), passes one barrier, refills the KPB slots
-// that iteration k0-KPB read with slices k0+KPB .., and runs its KPB slices,
-// so the copy wait, the barrier and the copy issue are paid once per KPB
-// slices instead of once per slice.  Same k order and accumulation as
-// mainloop.
+// Wait until the copies of at most min(newer, N) groups (L each) are in flight.
+template <int L, int N>
+__device__ __forceinline__ void wait_groups(int newer) {
+  if constexpr (N == 0) {
+    wait_vm<0>();
+  } else {
+    if (newer >= N)
+      wait_vm<N * L>();
+    else
+      wait_groups<L, N - 1>(newer);
+  }
+}
+
+// The operand fragments of one K slice, held in registers.
 template <class C>
-__device__ __forceinline__ void mainloop_multi(const f16* __restrict__ A,
-                                               const f16* __restrict__ W, int M, int K, int m0,
-                                               int n0, f16* smem, f32x16 (&acc)[C::FM][C::FN]) {
+struct Frags {
+  f16x8 a[C::BK / 16][C::FM], w[C::BK / 16][C::FN];
+  __device__ __forceinline__ void read(const f16* sA, const f16* sW, int wave) {
+    const int lane = threadIdx.x & 63, wm = wave / C::WN, wn = wave % C::WN;
+    const int r32 = lane & 31, kh = lane >> 5;
+#pragma unroll
+    for (int s = 0; s < C::BK / 16; ++s) {
+#pragma unroll
+      for (int fm = 0; fm < C::FM; ++fm)
+        a[s][fm] = *reinterpret_cast<const f16x8*>(
+            sA + C::L::off(wm * C::TM + fm * 32 + r32, 2 * s + kh));
+#pragma unroll
+      for (int fn = 0; fn < C::FN; ++fn)
+        w[s][fn] = *reinterpret_cast<const f16x8*>(
+            sW + C::L::off(wn * C::TN + fn * 32 + r32, 2 * s + kh));
+    }
+  }
+  __device__ __forceinline__ void mul(f32x16 (&acc)[C::FM][C::FN]) const {
+#pragma unroll
+    for (int s = 0; s < C::BK / 16; ++s)
+#pragma unroll
+      for (int fm = 0; fm < C::FM; ++fm)
+#pragma unroll
+        for (int fn = 0; fn < C::FN; ++fn)
+          acc[fm][fn] = mfma32(w[s][fn], a[s][fm], acc[fm][fn]);
+  }
+};
+
+// The K loop of tiles that have a CU to themselves (at most one workgroup per
+// CU), where nothing but the workgroup's own wavefronts can hide a stall.
+// A and W share one ring of R slices, filled R - KPB slices ahead, so a
+// slice's L2 latency is never exposed.  A 1 KB copy holds the wavefront that
+// issues it for ~16 cycles (the 64 B/clk of the texture path), and on a
+// wavefront that also computes that time adds to its LDS reads and MFMAs
+// instead of hiding behind them (FFN2 at 16 rows, 32-column tiles: 1.9 us of
+// copies and 1.2 us of reads and MFMAs over a fixed 3.7 us ran 7.2 us; 5.6 us
+// with one wavefront copying and one computing).  So NP wavefronts do the
+// copies and nothing else, and the others read slice kt's fragments while
+// the MFMAs of slice kt - 1 run.  One barrier per KPB slices: it publishes the
+// group that the copiers waited for and frees the group read before it.  Same
+// k order and accumulation as mainloop.
+template <class C>
+__device__ __forceinline__ void mainloop_deep(const f16* __restrict__ A,
+                                              const f16* __restrict__ W, int M, int K, int m0,
+                                              int n0, f16* smem, f32x16 (&acc)[C::FM][C::FN]) {
 #pragma unroll
   for (int fm = 0; fm < C::FM; ++fm)
 #pragma unroll
@@ -252,35 +309,69 @@ __device__ __forceinline__ void mainloop_multi(const f16* __restrict__ A,
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[fm][fn][i] = 0.f;
 
-  constexpr int P = C::KPB;
-  const int KT = K / C::BK;
+  constexpr int R = C::SA, P = C::KPB, G = R / P, L = C::LA + C::LW;
+  static_assert((G - 2) * P * L < 64, "vmcnt range");
+  const int KT = K / C::BK, wave = wave_id();
   f16* ringA = smem;
   f16* ringW = smem + C::W_BASE;
-  const f16* a0 = A + (size_t)m0 * K;
-  const f16* w0 = W + (size_t)n0 * K;
+  const int cw = C::NP > 0 ? wave - C::NW : wave;  // number among the copying wavefronts
+  const bool copies = C::NP == 0 || wave >= C::NW;
   uint32_t offA[C::LA], offW[C::LW];
-  row_offsets<C::BM, C::NW>(K, M - m0, offA);
-  row_offsets<C::BN, C::NW>(K, C::BN, offW);
-  const __amdgpu_buffer_rsrc_t rA = buffer_of(a0, (uint32_t)(M - m0) * K * 2u);
-  const __amdgpu_buffer_rsrc_t rW = buffer_of(w0, (uint32_t)C::BN * K * 2u);
-  auto issue = [&](int s) {
-    issue_rows_at<C::BN, C::NW>(rW, s * C::BK * 2, offW, ringW + (s % C::SW) * C::W_STAGE);
-    issue_rows_at<C::BM, C::NW>(rA, s * C::BK * 2, offA, ringA + (s % C::SA) * C::A_STAGE);
+  const __amdgpu_buffer_rsrc_t rA = buffer_of(A + (size_t)m0 * K, (uint32_t)(M - m0) * K * 2u);
+  const __amdgpu_buffer_rsrc_t rW = buffer_of(W + (size_t)n0 * K, (uint32_t)C::BN * K * 2u);
+  auto issue = [&](int s, int slot) {
+    issue_rows_at<C::BN, C::NC>(rW, s * C::BK * 2, offW, ringW + slot * C::W_STAGE, cw);
+    issue_rows_at<C::BM, C::NC>(rA, s * C::BK * 2, offA, ringA + slot * C::A_STAGE, cw);
   };
-#pragma unroll
-  for (int d = 0; d < P; ++d)
-    if (d < KT) issue(d);
-  for (int k0 = 0; k0 < KT; k0 += P) {
-    wait_vm<0>();
-    lds_barrier();  // slices k0 .. k0+P-1 visible to all; k0-P .. k0-1 consumed
+  int slot = 0;  // of slice kt
+  // Slices kt .. kt+P-1 landed: the copies of newer groups may be in flight (a
+  // last group of fewer than P slices counts for none, which only makes the
+  // wait stricter).
+  auto landed = [&](int kt) {
+    wait_groups<P * L, G - 2>(KT % P == 0 ? (KT - 1 - kt) / P : max(0, (KT - 1 - kt) / P - 1));
+  };
+  auto refill = [&](int kt) {  // the group R - P slices ahead, over the group read before this one
 #pragma unroll
     for (int d = 0; d < P; ++d)
-      if (k0 + P + d < KT) issue(k0 + P + d);
+      if (kt + R - P + d < KT) issue(kt + R - P + d, (slot + R - P + d) % R);
+  };
+  if (copies) {
+    row_offsets<C::BM, C::NC>(K, M - m0, offA, cw);
+    row_offsets<C::BN, C::NC>(K, C::BN, offW, cw);
 #pragma unroll
-    for (int d = 0; d < P; ++d)
-      if (k0 + d < KT)
-        compute_slice<C>(ringA + ((k0 + d) % C::SA) * C::A_STAGE,
-                         ringW + ((k0 + d) % C::SW) * C::W_STAGE, acc);
+    for (int d = 0; d < R - P; ++d)
+      if (d < KT) issue(d, d);
+  }
+  if (C::NP > 0 && copies) {
+    for (int kt = 0; kt < KT; kt += P) {
+      landed(kt);
+      lds_barrier();
+      refill(kt);
+      slot = (slot + P) % R;
+    }
+  } else {
+    Frags<C> f[2];
+    auto step = [&](int kt, Frags<C>& cur, const Frags<C>& prev) {
+      if (kt % P == 0) {
+        if constexpr (C::NP == 0) landed(kt);
+        lds_barrier();  // also this wavefront's reads of the slices before
+        if constexpr (C::NP == 0) refill(kt);
+      }
+      cur.read(ringA + slot * C::A_STAGE, ringW + slot * C::W_STAGE, wave);
+      slot = slot + 1 == R ? 0 : slot + 1;
+      if (kt > 0) prev.mul(acc);
+    };
+    int kt = 0;
+    for (; kt + 1 < KT; kt += 2) {
+      step(kt, f[0], f[1]);
+      step(kt + 1, f[1], f[0]);
+    }
+    if (kt < KT) {
+      step(kt, f[0], f[1]);
+      f[0].mul(acc);
+    } else {
+      f[1].mul(acc);
+    }
   }
   lds_barrier();  // ring free for the epilogue
 }
@@ -617,8 +708,8 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(
   f32x16 acc[C::FM][C::FN];
   if constexpr (C::PD > 0)
     mainloop_reg<C>(A, W, M, K, m0, n0, smem, acc);
-  else if constexpr (C::KPB > 1)
-    mainloop_multi<C>(A, W, M, K, m0, n0, smem, acc);
+  else if constexpr (C::DEEP)
+    mainloop_deep<C>(A, W, M, K, m0, n0, smem, acc);
   else
     mainloop<C>(A, W, M, K, m0, n0, smem, acc);
 
@@ -665,16 +756,18 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(
     }
     fcol = fc_lds;
     lds_barrier();
+    if (C::NP == 0 || wave < C::NW) {
 #pragma unroll
-    for (int fm = 0; fm < C::FM; ++fm) {
-      const int row = wm * C::TM + fm * 32 + r32;
-      mean[fm] = red[2 * row];
-      rstd[fm] = red[2 * row + 1];
+      for (int fm = 0; fm < C::FM; ++fm) {
+        const int row = wm * C::TM + fm * 32 + r32;
+        mean[fm] = red[2 * row];
+        rstd[fm] = red[2 * row + 1];
+      }
     }
   }
 
   if constexpr (EPI == kLayerNorm) {
-    static_assert(C::BN == kHidden, "LayerNorm tile owns whole 384-wide rows");
+    static_assert(C::BN == kHidden && C::NP == 0, "LayerNorm tile owns whole 384-wide rows");
     // v = acc + bias + residual, then the row statistics (lane ^ 32 holds the
     // other half of the wave's columns, LDS across wn).
     // The residual rows arrive through the (still free) output staging area:
@@ -765,13 +858,15 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(
     }
   }
 
+  // (The copying wavefronts of mainloop_deep hold no part of the tile; they
+  // take their share of the stores.)
   // fp16 tile into LDS (row pass p holds tile rows [p*PR, (p+1)*PR)), then
   // coalesced stores, which add the residual for kResidual (16-byte loads laid
   // out like the output rows).  One 32x32 block at a time; the scheduling
   // fence keeps a single block's values live.
 #pragma unroll
   for (int p = 0; p < C::NPASS; ++p) {
-    if (C::NPASS == 1 || wm == p) {
+    if ((C::NPASS == 1 || wm == p) && (C::NP == 0 || wave < C::NW)) {
 #pragma unroll
       for (int fn = 0; fn < C::FN; ++fn) {
         if constexpr (!kHoist) load_cols(fn, 0);
@@ -1542,7 +1637,7 @@ hipError_t launch(const f16* A, const f16* W, const f16* bias, const f16* residu
 }
 
 // Tile configurations (BM, BN, wavefronts M x N, A-ring depth), by id; the K
-// slice is 64 wide and the W ring 2 deep but in tile 34.  The product build holds
+// slice is 64 wide and the W ring 2 deep but in tiles 35-41.  The product build holds
 // the configurations pick_plain and gemm_residual_ln_tile choose; the others
 // of the sweep that chose them are compiled only with -DBBH_TUNING.
 //   id  tile      wave tile  SA   LDS
@@ -1558,8 +1653,15 @@ hipError_t launch(const f16* A, const f16* W, const f16* bias, const f16* residu
 //   30  128x128   64x32 (8w) PD 2   64 KB
 //   31  128x128   32x64 (8w) PD 2   64 KB
 //   32  128x192   32x96 (8w) PD 2   80 KB
-//   copy rings with two K slices per barrier (PD -2; A and W rings 4 deep):
-//   34  64x64     32x32      4/4    64 KB
+//   one workgroup per CU, A and W in one ring of SA slices (mainloop_deep),
+//   NP copying wavefronts:
+//   35  32x64     32x32 (2w) 6     72 KB   NP 4, two slices per barrier
+//   36  64x64     32x32      6     96 KB   NP 4, two slices per barrier
+//   37  96x64     32x32 (6w) 4     80 KB   NP 4
+//   38  128x64    32x32 (8w) 4     96 KB   NP 4
+//   39  96x128    32x64 (6w) 4    112 KB   NP 4
+//   40  128x128   64x64      4    128 KB   NP 4
+//   41  64x128    32x32 (8w) 3     72 KB   NP 0
 // Kernel symbols read gemm_kernel<Cfg<BM,BN,WM,WN,SA,PD,SW>, epilogue>.
 // The table itself: X(id, BM, BN, WM, WN, SA, PD, SW).
 #define BBH_TILES(X) \
@@ -1573,7 +1675,13 @@ hipError_t launch(const f16* A, const f16* W, const f16* bias, const f16* residu
   X(30, 128, 128, 2, 4, 2, 2, 2) \
   X(31, 128, 128, 4, 2, 2, 2, 2) \
   X(32, 128, 192, 4, 2, 2, 2, 2) \
-  X(34, 64, 64, 2, 2, 4, -2, 4)
+  X(35, 32, 64, 1, 2, 6, -66, 6) \
+  X(36, 64, 64, 2, 2, 6, -66, 6) \
+  X(37, 96, 64, 3, 2, 4, -65, 4) \
+  X(38, 128, 64, 4, 2, 4, -65, 4) \
+  X(39, 96, 128, 3, 2, 4, -65, 4) \
+  X(40, 128, 128, 2, 2, 4, -65, 4) \
+  X(41, 64, 128, 2, 4, 3, -1, 3)
 
 #ifdef BBH_TUNING
 // The rest of the sweep (ids 2-13, 15-17, 20-25, 27, 29).
@@ -1668,19 +1776,13 @@ const char* tile_name(int id) {
 // LDS traffic per MFMA).  Up to 4096 rows (the batch-64 forwards of the
 // length buckets) the best tile depends on whether other forwards share the
 // CUs.
-// Alone (shared false: bbh_embed, a one-slot pool), from sweeps of the
-// configs[1] and one-slot configs[3] forwards with one GEMM's tile changed at
-// a time: QKV runs the 64x64 copy-ring tile (0) up to 1024 rows (configs[1]
-// forward 230.1 -> 224.3 us: 288 workgroups instead of 72); FFN1 keeps that
-// tile to 4096 rows (with the LayerNorm carried in: one-slot pass 8.22-8.24
-// -> 8.11 ms against the register-staged 64x64 at 2049-3072 rows); O-proj
-// and FFN2 from 2049 rows run the 64x64 copy ring with two K slices per
-// barrier (34; one-slot varlen pass 9.00-9.03 -> 8.84-8.95 ms).  More
-// workgroups than CUs keep every CU busy, and the deeper rings fit beside
-// nothing else.  At 513-1024 rows alone FFN1 takes tile 34 (configs[1]
-// forward 195.4-195.8 -> 194.6-194.8 us, four interleaved repeats); at
-// 6145-8192 rows alone FFN1 takes tile 31, FFN2 tile 30 and O-proj tile 0
-// (configs[2] forward 387.5 -> 383.5 us on one box, every repeat; level on
+// Alone (shared false: bbh_embed, a one-slot pool), pick_deep's tiles first;
+// past them, from sweeps with one GEMM's tile changed at a time: QKV runs the
+// 64x64 copy-ring tile (0) up to 2048 rows (2048 rows: 6.4 us against 6.9 on
+// tile 30), FFN1 to 4096 rows (one-slot pass 8.22-8.24 -> 8.11 ms against the
+// register-staged 64x64 at 2049-3072 rows): more workgroups than CUs keep
+// every CU busy.  At 6145-8192 rows alone FFN1 takes tile 31 and O-proj tile
+// 0 (configs[2] forward 387.5 -> 383.5 us on one box, every repeat; level on
 // a slower one).
 // Beside other forwards (shared true: a pool of several slots) every tile was
 // tried for each (shape, M) with the others fixed in the per-batch pass, then
@@ -1696,17 +1798,47 @@ const char* tile_name(int id) {
 // four repeats each; alone they are slower there).
 // There the other forwards fill the CUs, and fewer, larger tiles move fewer
 // bytes L2 -> CU per FLOP.
+// Alone, where one workgroup per CU covers the output (kCus CUs): the smallest
+// of the mainloop_deep tiles that needs at most kCus workgroups.  Such a
+// GEMM is bound by one workgroup's walk over K, which a smaller tile
+// shortens (fewer bytes through its CU per slice); one workgroup more than
+// CUs would start a second round.  Against the tiles that ran before, back to
+// back launches on one box: FFN2 at 16 / 1024 / 2048 / 3072 / 4096 / 6144 /
+// 8192 rows 9.6 / 10.3 / 10.5 / 11.4 / 12.0 / 16.1 / 17.6 -> 5.7 / 6.1 / 7.1 /
+// 8.6 / 10.0 / 12.4 / 15.6 us; O-proj at 16 / 1024 / 2048 / 3072 / 4096 rows
+// 4.0 / 4.4 / 4.5 / 4.9 / 5.1 -> 2.9 / 3.2 / 3.7 / 4.5 / 4.8; FFN1 at 16 /
+// 256 / 1024 rows 5.1 / 5.7 / 6.5 -> 4.0 / 4.9 / 5.7; QKV at 16 / 1024 rows
+// 4.7 / 5.5 -> 3.5 / 5.0.  With K < 1024 the tiles above 64x128 no longer gain
+// (six slices: the epilogue, not the walk, grows).  An empty kernel takes
+// 1.65 us in such a stream.  -1: none.
+constexpr int kCus = 256;
+int pick_deep(int M, int N, int K) {
+  const bool wide_k = K >= 1024;
+  struct Tile {
+    int id, bm, bn;
+  };
+  static constexpr Tile wide[] = {{35, 32, 64},  {36, 64, 64},  {37, 96, 64},
+                                  {38, 128, 64}, {39, 96, 128}, {40, 128, 128}};
+  static constexpr Tile narrow[] = {{35, 32, 64}, {36, 64, 64}, {37, 96, 64}, {41, 64, 128}};
+  const Tile* t = wide_k ? wide : narrow;
+  for (int i = 0; i < (wide_k ? 6 : 4); ++i)
+    if (N % t[i].bn == 0 && (long)((M + t[i].bm - 1) / t[i].bm) * (N / t[i].bn) <= kCus)
+      return t[i].id;
+  return -1;
+}
+
 int pick_plain(int M, int N, int K, bool shared) {
   const bool qkv = N == 1152, ffn1 = N == 1536, wide_k = K >= 1024;
-  int id;
+  int id = shared ? -1 : pick_deep(M, N, K);
+  if (id >= 0) return id;
   if (M <= 1024)
-    id = qkv ? (shared ? 30 : 0) : ffn1 ? (!shared && M > 512 ? 34 : 0) : 26;
+    id = qkv ? (shared ? 30 : 0) : ffn1 ? 0 : shared ? 26 : 0;
   else if (M <= 2048)
-    id = qkv ? 30 : ffn1 ? (shared ? 30 : 0) : !shared ? 26 : wide_k ? 1 : 30;
+    id = !shared ? 0 : wide_k ? 1 : 30;
   else if (M <= 3072)
-    id = qkv ? 30 : ffn1 ? (shared ? 30 : 0) : !shared ? 34 : wide_k ? 1 : 30;
+    id = qkv ? 30 : ffn1 ? (shared ? 30 : 0) : !shared ? 0 : wide_k ? 1 : 30;
   else if (M <= 4096)
-    id = qkv ? (shared ? 30 : 32) : ffn1 ? (shared ? 30 : 0) : !shared ? 34 : wide_k ? 1 : 30;
+    id = qkv ? (shared ? 30 : 32) : ffn1 ? (shared ? 30 : 0) : !shared ? 0 : wide_k ? 1 : 30;
   else if (M <= 6144)
     id = qkv ? 30 : ffn1 ? 26 : wide_k ? 31 : 0;
   else if (M <= 8192)
@@ -1797,7 +1929,13 @@ hipError_t launch_carry(int id, const f16* A, const f16* W, const f16* bias, con
     BBH_CARRY(30)
     BBH_CARRY(31)
     BBH_CARRY(32)
-    BBH_CARRY(34)
+    BBH_CARRY(35)
+    BBH_CARRY(36)
+    BBH_CARRY(37)
+    BBH_CARRY(38)
+    BBH_CARRY(39)
+    BBH_CARRY(40)
+    BBH_CARRY(41)
   }
 #undef BBH_CARRY
   return hipErrorInvalidValue;

@@ -31,7 +31,7 @@ GEMM_SHAPES = [
     (4096, 384, 1536, False), (100, 128, 64, False), (7, 64, 128, True),
     # the batch-64 buckets' tiles, ragged: 128x128 for FFN1, 64x128 for FFN2
     (2500, 1536, 384, True), (3000, 384, 1536, False),
-    # two K slices per barrier (tile 34) with an odd slice count (3, 1)
+    # odd slice counts (3, 1)
     (3000, 384, 192, False), (2100, 384, 64, True),
     # large-M tiles (cfg5 runs M = 131072 end to end), one shape per tile bucket
     (12288, 1152, 384, False), (16384, 384, 1536, False),
@@ -65,7 +65,7 @@ def test_linear_rows_identical_across_kernels(torch_cuda, N, gelu):
     # every kernel accumulates in the same k order and rounds the same way.
     # M = 50000 runs QKV and FFN1 on the weight-resident kernel and N = 384 on
     # a 128x128 tile; M = 2048 runs all three on 64x64 tiles; M = 3000 runs
-    # N = 384 on the 64x64 copy ring with two K slices per barrier (tile 34).
+    # N = 384 below and above one workgroup per CU.
     torch = torch_cuda
     from bbh import engine
 
@@ -346,6 +346,34 @@ def test_unfused_attention_pieces_match_fused(torch_cuda):
     fused = torch.empty_like(merged)
     engine.launch_attention(tq, tm, fused, B, S)
     assert np.abs(_np(fused) - _np(merged)).max() <= TOL
+
+
+@pytest.mark.parametrize("N,K,Ms", [
+    # The one-workgroup-per-CU tiles: at most 256 workgroups of 32x64, 64x64,
+    # 96x64, 128x64, 96x128 and 128x128 (K >= 1024), each at its last row count
+    # and one past it; 17 slices leave a part-filled group of two.
+    (384, 1536, (1, 33, 1344, 1345, 2688, 2689, 4032, 4033, 5376, 5377, 8160, 8161)),
+    (384, 1088, (16, 2500)), (64, 1024, (8000,)),
+    # K < 1024: 32x64, 64x64, 96x64, 64x128; three slices, one slice.
+    (384, 384, (16, 1345, 2689, 4033, 5440)), (1536, 384, (320, 321, 641, 961, 1344, 1345)),
+    (1152, 192, (31, 449)), (128, 64, (1, 4097))])
+def test_linear_rows_do_not_depend_on_the_tile(torch_cuda, N, K, Ms):
+    # Every tile adds k in the same order and rounds the same way: the rows of
+    # any row count are, bit for bit, those of a call with 50000 rows.
+    torch = torch_cuda
+    from bbh import engine
+
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    A = torch.randn((50000, K), device="cuda", generator=g).half()
+    W = (torch.randn((N, K), device="cuda", generator=g) / K ** 0.5).half()
+    b = (torch.randn((N,), device="cuda", generator=g) * 0.1).half()
+    ref = torch.empty((50000, N), dtype=torch.float16, device="cuda")
+    engine.launch_matmul(A, W, ref, 50000, N, K, bias=b)
+    for M in Ms:
+        C = torch.full((M + 1, N), 7.0, dtype=torch.float16, device="cuda")
+        engine.launch_matmul(A, W, C, M, N, K, bias=b)
+        assert torch.equal(C[:M], ref[:M]), M
+        assert torch.all(C[M] == 7.0)  # nothing past the last row
 
 
 @pytest.mark.parametrize("B,S,off", [(1, 16, 0), (3, 48, 1), (2, 80, 0), (2, 128, 3), (1, 144, 0),
