@@ -230,22 +230,32 @@ def launch_work(r):
     return flops, byts
 
 
-def qkv_attention_rows(seq):
-    """Rows of a qkv_attention_kernel workgroup at this sentence length: 192 (six
-    wavefronts) for seq 48, 80 and 96, whose sentences fill 192 rows exactly, else 128."""
-    return 192 if seq in (48, 80, 96) else 128
+def qkv_attention_rows(batch, seq, shared=False):
+    """Rows of a qkv_attention_kernel workgroup, the first template argument of
+    its kernel symbol (the launcher's rule): alone the smallest of 64 / 128 /
+    192 / 256 rows that gives at most one workgroup per CU, past that 128 or
+    192, whichever takes fewer rounds of two workgroups a CU times rows;
+    beside other forwards 192 for seq 48, 80 and 96, else 128."""
+    if shared:
+        return 192 if seq in (48, 80, 96) else 128
+    wgs = lambda rows: 12 * -(-batch // (rows // seq))  # noqa: E731
+    for rows in (64, 128, 192, 256):
+        if rows >= seq and wgs(rows) <= 256:
+            return rows
+    cost = lambda rows: -(-wgs(rows) // 512) * rows  # noqa: E731
+    return 128 if cost(128) < cost(192) else 192
 
 
-def kernel_name(engine, op, tile, fused, seq=0):
-    """(display name, class name as short_kernel() writes it) of a launch record;
-    seq: the sentence length of a fused QKV + attention record (its k)."""
+def kernel_name(engine, op, tile, fused, batch=0, seq=0):
+    """(display name, class name as short_kernel() writes it) of a launch record
+    of a forward alone; batch, seq: of a fused QKV + attention record (n, k)."""
     row = {"attention": "attention_kernel", "embed": "embedding_ln_kernel",
            "pool": "pool_normalize_kernel", "layernorm": "ln384_kernel",
            "ffn": "ffn_fused_kernel"}
     if op in row:
         return row[op], row[op]
     if op == "qkv" and fused == 3:
-        name = f"qkv_attention_kernel<{qkv_attention_rows(seq)}>"
+        name = f"qkv_attention_kernel<{qkv_attention_rows(batch, seq)}>"
         return name, name
     if fused == 2:  # the LayerNorm carried between the GEMMs as row statistics
         epi = {"qkv": "4 (carried LayerNorm in)", "ffn1_gelu": "5 (carried LayerNorm in+GELU)"}.get(
@@ -259,16 +269,19 @@ def kernel_name(engine, op, tile, fused, seq=0):
 
 
 def gemm_grid_items(tile_name, M, N):
-    """Work-items of a tiled-GEMM launch (the launcher's grid: N/BN column
-    tiles x 8 XCDs x ceil(M-tiles / 8), 64*WM*WN threads), as rocprofv3
+    """Work-items of a tiled-GEMM launch (the launcher's grid: the tiles dealt to
+    8 XCDs, or to one XCD a row of tiles below 8 rows of at most 32 tiles;
+    64 threads for each computing and each copying wavefront), as rocprofv3
     reports Grid_Size; None for other kernels."""
     import re
 
-    m = re.match(r"Cfg<(\d+),(\d+),(\d+),(\d+),", tile_name)
+    m = re.match(r"Cfg<(\d+),(\d+),(\d+),(\d+),(\d+),(-?\d+),", tile_name)
     if not m:
         return None
-    bm, bn, wm, wn = (int(x) for x in m.groups())
-    return (N // bn) * 8 * ((-(-M // bm) + 7) // 8) * 64 * wm * wn
+    bm, bn, wm, wn, _, pd = (int(x) for x in m.groups())
+    rows, cols = -(-M // bm), N // bn
+    xcds = rows if rows < 8 and cols <= 32 else 8
+    return -(-rows * cols // xcds) * 8 * 64 * (wm * wn + (-pd // 16 if pd < 0 else 0))
 
 
 def classify(engine, recs, steps):
@@ -276,7 +289,7 @@ def classify(engine, recs, steps):
     algorithmic FLOPs and bytes, sorted by summed time."""
     classes = {}
     for r in recs:
-        key = (r["op"], r["tile"], r["fused_ln"], r["m"], r["k"] if r["fused_ln"] == 3 else 0)
+        key = (r["op"], r["tile"], r["fused_ln"], r["m"], (r["n"], r["k"]) if r["fused_ln"] == 3 else (0, 0))
         c = classes.setdefault(key, {"ms": 0.0, "n": 0, "flops": 0.0, "bytes": 0.0, "m": set()})
         f, b = launch_work(r)
         c["ms"] += r["ms"]
@@ -286,9 +299,9 @@ def classify(engine, recs, steps):
         c["bytes"] += b
     total = sum(c["ms"] for c in classes.values())
     rows = []
-    for (op, tile, fused, m, seq), c in sorted(classes.items(), key=lambda kv: -kv[1]["ms"]):
+    for (op, tile, fused, m, (batch, seq)), c in sorted(classes.items(), key=lambda kv: -kv[1]["ms"]):
         avg_s = c["ms"] / c["n"] / 1e3
-        name, cls = kernel_name(engine, op, tile, fused, seq)
+        name, cls = kernel_name(engine, op, tile, fused, batch, seq)
         n_out = {"qkv": 1152, "ffn1_gelu": 1536}.get(op, 384)
         grid = gemm_grid_items(engine.gemm_tile_name(tile), m, n_out) if tile >= 0 else None
         rows.append({"kernel": name, "class": cls, "op": op, "m": m, "grid_items": grid,

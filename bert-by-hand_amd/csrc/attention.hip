@@ -86,11 +86,12 @@ __global__ __launch_bounds__(64 * NW, T == 2 ? 4 : 6) void attention_kernel(
     const f16* __restrict__ qkv, const int32_t* __restrict__ mask, f16* __restrict__ out,
     int batch, int seq, int heads, float c, const PackedSentence* __restrict__ sents) {
   HIP_DYNAMIC_SHARED(f16, smem);
-  // (sequence, head) of this workgroup; all heads of a sequence go to one XCD
-  // (workgroup id % 8) back to back, so its QKV rows are fetched into one L2.
-  const int x = blockIdx.x & 7, k = blockIdx.x >> 3;
-  const int b = (k / heads) * 8 + x, h = k % heads;
-  if (b >= batch) return;
+  // (sequence, head) of this workgroup; the heads of a sequence go to one XCD
+  // back to back (but where its span ends), so its QKV rows are fetched into
+  // one L2.
+  const int item = xcd_item(batch, heads);
+  if (item < 0) return;
+  const int b = item / heads, h = item - b * heads;
   size_t row0 = (size_t)b * seq;  // first hidden row of the sentence
   if constexpr (VL) {
     const PackedSentence sn = sents[b];
@@ -322,7 +323,7 @@ hipError_t launch_attention(const f16* qkv, const int32_t* mask, f16* merged, in
       reinterpret_cast<const void*>(attention_kernel<NW, T, F, VL>),
       hipFuncAttributeMaxDynamicSharedMemorySize, (int)attn_lds_bytes(kMaxPos, NW * T));
   if (attr != hipSuccess) return attr;
-  const int grid = heads * 8 * ((batch + 7) / 8);
+  const int grid = xcd_grid(batch, heads);
   hipLaunchKernelGGL((attention_kernel<NW, T, F, VL>), dim3(grid), dim3(64 * NW),
                      attn_lds_bytes(seq, staged), s, qkv, mask, merged, batch, seq, heads, c,
                      sents);

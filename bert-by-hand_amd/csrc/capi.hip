@@ -607,7 +607,7 @@ bbh_status run_layers_carried(bbh_workspace* ws, const bbh_model* m, f16* h0, co
       BBH_TRY(timed_op(t, s, {BBH_OP_QKV, -1, 3, M, segs[0].batch, segs[0].seq, 0.f}, [&] {
         return check_launch(bbh::qkv_attention(cur, L.qkv_wp, L.qkv_fsp, L.qkv_fcp, cy,
                                                segs[0].mask, ws->ctx, segs[0].batch,
-                                               segs[0].seq, kScale, eps, s),
+                                               segs[0].seq, kScale, eps, s, sh),
                             "qkv + attention");
       }));
     } else if (!P) {

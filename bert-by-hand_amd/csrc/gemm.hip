@@ -457,10 +457,10 @@ __device__ __forceinline__ void mainloop_reg(const f16* __restrict__ A,
 
 // Tile coordinates from the workgroup id, XCD-aware (see header).
 __device__ __forceinline__ bool tile_of(int nb, int mb, int& mi, int& ni) {
-  const int b = blockIdx.x, x = b & 7, k = b >> 3;
-  ni = k % nb;
-  mi = (k / nb) * 8 + x;
-  return mi < mb;
+  const int t = xcd_item(mb, nb);
+  mi = t / nb;
+  ni = t - mi * nb;
+  return t >= 0;
 }
 
 // Write ROWS rows of the output tile, staged in LDS as ROWS x OUT_LD fp16,
@@ -920,7 +920,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(
 // A batch-64 forward spends about a tenth of its time in attention launches
 // whose work is a few hundred cycles: one global round trip for Q, K and V
 // just written by the QKV Linear, then the launch's tail.  Here workgroup
-// (group of G = 128 / seq sentences, head h) computes the QKV Linear's 96
+// (group of G = BM / seq sentences, head h) computes the QKV Linear's 96
 // columns of head h over the group's rows (a head-major copy of W: rows
 // h*96 .. h*96+95 are Q, K, V of head h), with the bias or carried-LayerNorm
 // epilogue of gemm_fold, writes them to LDS as Q rows, K rows (the attention
@@ -930,30 +930,29 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(
 namespace qa {
 constexpr int HD = kHeadDim, NQ = 3 * HD;
 constexpr float kLazy = 8.f;  // as attention_kernel: the running max may lag by 2^8
-// A workgroup of BM / 32 wavefronts over BM rows (128, or 192 where a
-// sentence length fills it better).  LDS after the K loop (bytes): Q
+// A workgroup over BM rows: BM / 32 x WN computing wavefronts (WN = 1: all 96
+// columns; 3: one of Q, K, V) and NP copying ones, a ring of R slices
+// (mainloop_deep); all of them attend.  LDS after the K loop (bytes): Q
 // [BM][32], K [KR][32] (swizzled), V^T [32][VLD], key bias [G][round32(seq)]
 // (at most 2 BM), row (mean, rstd) [BM], fs / fc [2][96], and each
-// wavefront's 32 x 32 output tile [32][kOutLd] (all within the K loop's ring).
+// wavefront's 32 x 32 output tile [32][kOutLd].
 constexpr int kOutLd = 40;  // halves per row of a wavefront's output tile
-template <int BM_>
+template <int BM_, int WN, int R, int NP>
 struct Layout {
-  static constexpr int BM = BM_, NWV = BM / 32, NT = 64 * NWV, KR = BM + 32, VLD = KR + 8;
-  static constexpr int MBN = 2 * BM;  // >= G * round32(seq) for every seq, = NT
-  using C = Cfg<BM, NQ, NWV, 1, 2, 0, 2>;
+  using C = Cfg<BM_, NQ, BM_ / 32, WN, R, -(16 * NP + 1), R>;
+  static constexpr int BM = BM_, NWV = C::NW + C::NP, NT = C::THREADS, KR = BM + 32, VLD = KR + 8;
+  static constexpr int MBN = 2 * BM;  // >= G * round32(seq) for every seq
   static constexpr size_t OFF_Q = 0, OFF_K = OFF_Q + (size_t)BM * HD * 2,
-                          OFF_V = OFF_K + (size_t)KR * HD * 2, OFF_B = OFF_V + (size_t)HD * VLD * 2,
+                          OFF_V = OFF_K + (size_t)KR * HD * 2,
+                          OFF_B = OFF_V + (size_t)HD * VLD * 2,
                           OFF_R = OFF_B + (size_t)MBN * 4, OFF_F = OFF_R + (size_t)BM * 8,
                           OFF_S = (OFF_F + (size_t)2 * NQ * 4 + 15) & ~(size_t)15,
                           END = OFF_S + (size_t)NWV * 32 * kOutLd * 2;
   static constexpr size_t LDS = C::LDS > END ? C::LDS : END;
   static_assert(OFF_V % 16 == 0 && OFF_R % 16 == 0 && OFF_F % 16 == 0 && (VLD * 2) % 16 == 0,
                 "align");
-  static_assert(NT >= BM && NT >= NQ, "a thread per tile row / column");
+  static_assert(NT >= MBN && NT >= NQ, "a thread per key bias and column");
 };
-// Rows a workgroup takes for a sentence length: 192 where 128 would leave a
-// quarter or more of the tile idle (seq 48, 80, 96).
-inline int rows_for(int seq) { return (seq == 48 || seq == 80 || seq == 96) ? 192 : 128; }
 __device__ __forceinline__ int key_of_row(int r) {
   const int a = r >> 3, c = (r >> 2) & 1, b = r & 3;
   return 16 * (a >> 1) + 8 * c + 4 * (a & 1) + b;
@@ -961,20 +960,19 @@ __device__ __forceinline__ int key_of_row(int r) {
 __device__ __forceinline__ int ks_off(int key, int c) { return key * 32 + ((c ^ ((key >> 2) & 3)) << 3); }
 }  // namespace qa
 
-template <int BM_>
-__global__ __launch_bounds__(2 * BM_) void qkv_attention_kernel(
+template <int BM_, int WN_, int R_, int NP_>
+__global__ __launch_bounds__(64 * (BM_ / 32 * WN_ + NP_)) void qkv_attention_kernel(
     const f16* __restrict__ X, const f16* __restrict__ Wp, const float* __restrict__ fs,
     const float* __restrict__ fc, LnCarry cy, const int32_t* __restrict__ mask,
     f16* __restrict__ ctx, int batch, int seq, int G, float c, float eps) {
   using namespace qa;
-  using L = Layout<BM_>;
+  using L = Layout<BM_, WN_, R_, NP_>;
   using C = typename L::C;
   constexpr int BM = L::BM, KR = L::KR, VLD = L::VLD, NT = L::NT;
   HIP_DYNAMIC_SHARED(f16, smem);
-  const int x = blockIdx.x & 7, kx = blockIdx.x >> 3;
-  const int grp = (kx / kHeads) * 8 + x, h = kx % kHeads;
-  const int b0 = grp * G;
-  if (b0 >= batch) return;  // the whole workgroup: no barrier reached
+  const int item = xcd_item((batch + G - 1) / G, kHeads);
+  if (item < 0) return;  // the whole workgroup: no barrier reached
+  const int b0 = item / kHeads * G, h = item % kHeads;
   const int gv = min(G, batch - b0), M = batch * seq, m0 = b0 * seq, R = gv * seq;
   const int ntq = (seq + 31) >> 5, KP = ntq * 32;  // query tiles (key chunks) per sentence
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r32 = lane & 31, kh = lane >> 5;
@@ -1004,8 +1002,8 @@ __global__ __launch_bounds__(2 * BM_) void qkv_attention_kernel(
     if (key < seq) mv = mask[(size_t)(b0 + g) * seq + key];
   }
 
-  f32x16 acc[1][3];
-  mainloop<C>(X, Wp, M, kHidden, m0, h * NQ, smem, acc);
+  f32x16 acc[1][C::FN];
+  mainloop_deep<C>(X, Wp, M, kHidden, m0, h * NQ, smem, acc);
 
   unsigned char* lds = reinterpret_cast<unsigned char*>(smem);
   f16* Qs = reinterpret_cast<f16*>(lds + L::OFF_Q);
@@ -1034,31 +1032,33 @@ __global__ __launch_bounds__(2 * BM_) void qkv_attention_kernel(
     Vt[(i / (KR - BM)) * VLD + BM + i % (KR - BM)] = (f16)0.f;
   }
   lds_barrier();
-  {
-    // Epilogue: acc[0][fn][4j+e] is column fn*32 + 8j + 4kh + e (Q, K, V of
-    // head h) of local row r, as gemm_fold computes it.
-    const int r = wave * 32 + r32;
+  if (C::NP == 0 || wave < C::NW) {
+    // Epilogue: acc[0][fn][4j+e] is column 8j + 4kh + e of a part (Q, K or V
+    // of head h) of local row r, as gemm_fold computes it.
+    const int r = (wave / C::WN) * 32 + r32;
     const float2 st = rs[r];
 #pragma unroll
-    for (int fn = 0; fn < 3; ++fn)
+    for (int fn = 0; fn < C::FN; ++fn) {
+      const int part = (wave % C::WN) * C::FN + fn;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int d0 = 8 * j + 4 * kh;
-        const f32x4 sv = *reinterpret_cast<const f32x4*>(fcol + fn * HD + d0);
-        const f32x4 cv = *reinterpret_cast<const f32x4*>(fcol + NQ + fn * HD + d0);
+        const f32x4 sv = *reinterpret_cast<const f32x4*>(fcol + part * HD + d0);
+        const f32x4 cv = *reinterpret_cast<const f32x4*>(fcol + NQ + part * HD + d0);
         f16x4 o;
 #pragma unroll
         for (int e = 0; e < 4; ++e)
           o[e] = to_half(fmaf(-st.x, sv[e], acc[0][fn][4 * j + e]) * st.y + cv[e]);
-        if (fn == 0) {
+        if (part == 0) {
           *reinterpret_cast<f16x4*>(Qs + r * HD + d0) = o;
-        } else if (fn == 1) {
+        } else if (part == 1) {
           *reinterpret_cast<f16x4*>(Ks + ks_off(r, j) + 4 * kh) = o;
         } else {
 #pragma unroll
           for (int e = 0; e < 4; ++e) Vt[(d0 + e) * VLD + r] = o[e];
         }
       }
+    }
   }
   lds_barrier();
 
@@ -1188,8 +1188,7 @@ __global__ __launch_bounds__(2 * BM_) void qkv_attention_kernel(
     }
   };
   // Two-tile sentences (seq 33 .. 64) a wavefront each where one tile per
-  // wavefront would take two rounds (seq 48 on 192 rows: 8 tiles, 6
-  // wavefronts); otherwise one tile per wavefront.
+  // wavefront would take two rounds; otherwise one tile per wavefront.
   // Seq 16: two sentences a 32-row tile (queries and keys 0-15 of sentence
   // g0, 16-31 of g0 + 1) with the cross-sentence pairs masked, so half the
   // tiles.  A query's probabilities and sums are those of its own sentence's
@@ -1620,13 +1619,12 @@ hipError_t launch(const f16* A, const f16* W, const f16* bias, const f16* residu
     for (int r0 = 0; r0 < M; r0 += step) {
       const int mr = std::min(step, M - r0);
       const int nb = N / C::BN, mb = (mr + C::BM - 1) / C::BM;
-      const int grid = nb * 8 * ((mb + 7) / 8);
       LnCarry cr = cy;  // row-indexed like A and out
       if (cr.st_in) cr.st_in += (size_t)r0 * kMaxCarryTiles;
       if (cr.mr_out) cr.mr_out += r0;
       if (cr.mr_in) cr.mr_in += r0;
       if (cr.st_out) cr.st_out += (size_t)r0 * kMaxCarryTiles;
-      hipLaunchKernelGGL((gemm_kernel<C, EPI>), dim3(grid), dim3(C::THREADS), C::LDS, s,
+      hipLaunchKernelGGL((gemm_kernel<C, EPI>), dim3(xcd_grid(mb, nb)), dim3(C::THREADS), C::LDS, s,
                          A + (size_t)r0 * K, W, bias, residual ? residual + (size_t)r0 * N : nullptr,
                          gamma, beta, out + (size_t)r0 * N, mr, N, K, eps, cr);
       const hipError_t e = hipGetLastError();
@@ -1642,7 +1640,6 @@ hipError_t launch(const f16* A, const f16* W, const f16* bias, const f16* residu
 // of the sweep that chose them are compiled only with -DBBH_TUNING.
 //   id  tile      wave tile  SA   LDS
 //    0  64x64     32x32      4    48 KB
-//    1  64x128    32x64      4    64 KB
 //   14  64x384    64x96      2   112 KB   (owns whole 384-wide rows)
 //   8 wavefronts (2 per SIMD):
 //   18  128x384   64x96      4   160 KB   (owns whole rows)
@@ -1666,7 +1663,6 @@ hipError_t launch(const f16* A, const f16* W, const f16* bias, const f16* residu
 // The table itself: X(id, BM, BN, WM, WN, SA, PD, SW).
 #define BBH_TILES(X) \
   X(0, 64, 64, 2, 2, 4, 0, 2) \
-  X(1, 64, 128, 2, 2, 4, 0, 2) \
   X(14, 64, 384, 1, 4, 2, 0, 2) \
   X(18, 128, 384, 2, 4, 4, 0, 2) \
   X(19, 256, 192, 4, 2, 3, 0, 2) \
@@ -1684,8 +1680,9 @@ hipError_t launch(const f16* A, const f16* W, const f16* bias, const f16* residu
   X(41, 64, 128, 2, 4, 3, -1, 3)
 
 #ifdef BBH_TUNING
-// The rest of the sweep (ids 2-13, 15-17, 20-25, 27, 29).
+// The rest of the sweep (ids 1-13, 15-17, 20-25, 27, 29).
 #define BBH_TUNING_TILES(X) \
+  X(1, 64, 128, 2, 2, 4, 0, 2) \
   X(2, 128, 64, 2, 2, 4, 0, 2) \
   X(3, 128, 128, 2, 2, 4, 0, 2) \
   X(4, 256, 128, 2, 2, 3, 0, 2) \
@@ -1795,7 +1792,9 @@ const char* tile_name(int id) {
 // with QKV inside the attention kernel, O-proj to the 128x128 tile (30):
 // 4.117-4.127 -> 4.092-4.104 ms; FFN2 on tile 1 and O-proj on tile 30 from
 // 1025 rows as well (3.708 -> 3.668 ms, then 3.845-3.857 -> 3.828-3.843 ms,
-// four repeats each; alone they are slower there).
+// four repeats each; alone they are slower there).  With copying wavefronts
+// FFN2 takes tile 40 and O-proj tile 41 from 1025 rows (pass 3.933 -> 3.877 ->
+// 3.864 ms; the tiles with 96 KB and more of LDS, 36-39, +2.7 to +5.5%).
 // There the other forwards fill the CUs, and fewer, larger tiles move fewer
 // bytes L2 -> CU per FLOP.
 // Alone, where one workgroup per CU covers the output (kCus CUs): the smallest
@@ -1809,8 +1808,8 @@ const char* tile_name(int id) {
 // 4.0 / 4.4 / 4.5 / 4.9 / 5.1 -> 2.9 / 3.2 / 3.7 / 4.5 / 4.8; FFN1 at 16 /
 // 256 / 1024 rows 5.1 / 5.7 / 6.5 -> 4.0 / 4.9 / 5.7; QKV at 16 / 1024 rows
 // 4.7 / 5.5 -> 3.5 / 5.0.  With K < 1024 the tiles above 64x128 no longer gain
-// (six slices: the epilogue, not the walk, grows).  An empty kernel takes
-// 1.65 us in such a stream.  -1: none.
+// but at N = 384 (six slices: the epilogue, not the walk, grows).  An empty
+// kernel takes 1.65 us in such a stream.  -1: none.
 constexpr int kCus = 256;
 int pick_deep(int M, int N, int K) {
   const bool wide_k = K >= 1024;
@@ -1819,9 +1818,10 @@ int pick_deep(int M, int N, int K) {
   };
   static constexpr Tile wide[] = {{35, 32, 64},  {36, 64, 64},  {37, 96, 64},
                                   {38, 128, 64}, {39, 96, 128}, {40, 128, 128}};
-  static constexpr Tile narrow[] = {{35, 32, 64}, {36, 64, 64}, {37, 96, 64}, {41, 64, 128}};
+  static constexpr Tile narrow[] = {{35, 32, 64}, {36, 64, 64}, {37, 96, 64}, {41, 64, 128},
+                                    {39, 96, 128}};
   const Tile* t = wide_k ? wide : narrow;
-  for (int i = 0; i < (wide_k ? 6 : 4); ++i)
+  for (int i = 0; i < (wide_k ? 6 : N <= 384 ? 5 : 4); ++i)
     if (N % t[i].bn == 0 && (long)((M + t[i].bm - 1) / t[i].bm) * (N / t[i].bn) <= kCus)
       return t[i].id;
   return -1;
@@ -1834,15 +1834,15 @@ int pick_plain(int M, int N, int K, bool shared) {
   if (M <= 1024)
     id = qkv ? (shared ? 30 : 0) : ffn1 ? 0 : shared ? 26 : 0;
   else if (M <= 2048)
-    id = !shared ? 0 : wide_k ? 1 : 30;
+    id = !shared ? 0 : wide_k ? 40 : N == 384 ? 41 : 30;
   else if (M <= 3072)
-    id = qkv ? 30 : ffn1 ? (shared ? 30 : 0) : !shared ? 0 : wide_k ? 1 : 30;
+    id = qkv ? 30 : ffn1 ? (shared ? 30 : 0) : !shared ? 0 : wide_k ? 40 : 41;
   else if (M <= 4096)
-    id = qkv ? (shared ? 30 : 32) : ffn1 ? (shared ? 30 : 0) : !shared ? 0 : wide_k ? 1 : 30;
+    id = qkv ? (shared ? 30 : 32) : ffn1 ? (shared ? 30 : 0) : !shared ? 0 : wide_k ? 40 : 41;
   else if (M <= 6144)
-    id = qkv ? 30 : ffn1 ? 26 : wide_k ? 31 : 0;
+    id = qkv ? 30 : ffn1 ? (shared ? 26 : 19) : wide_k ? 31 : 0;
   else if (M <= 8192)
-    id = shared ? (wide_k ? 31 : 30) : qkv ? 30 : ffn1 ? 31 : wide_k ? 30 : 0;
+    id = shared ? (wide_k ? 31 : 30) : qkv || ffn1 ? 19 : wide_k ? 30 : 0;
   else if (M <= 16384)
     id = wide_k ? 32 : 30;
   else if (M <= 49152)
@@ -1924,7 +1924,7 @@ hipError_t launch_carry(int id, const f16* A, const f16* W, const f16* bias, con
     return launch<TileCfg<ID>, EPI>(A, W, bias, residual, gamma, beta, out, M, N, K, eps, s, cy);
   switch (id) {
     BBH_CARRY(0)
-    BBH_CARRY(1)
+    BBH_CARRY(19)
     BBH_CARRY(26)
     BBH_CARRY(30)
     BBH_CARRY(31)
@@ -1943,20 +1943,43 @@ hipError_t launch_carry(int id, const f16* A, const f16* W, const f16* bias, con
 
 bool ln_carry_ok(int M) { return M >= 1 && M <= 8192; }
 
-template <int BM>
+template <int BM, int WN, int R, int NP>
 hipError_t launch_qkv_attention(const f16* X, const f16* Wp, const float* fs, const float* fc,
                                 const LnCarry& cy, const int32_t* mask, f16* ctx, int batch, int seq,
                                 float c, float eps, hipStream_t s) {
-  using L = qa::Layout<BM>;
+  using L = qa::Layout<BM, WN, R, NP>;
   static const hipError_t attr =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(qkv_attention_kernel<BM>),
+      hipFuncSetAttribute(reinterpret_cast<const void*>(qkv_attention_kernel<BM, WN, R, NP>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)L::LDS);
   if (attr != hipSuccess) return attr;
   const int G = BM / seq, groups = (batch + G - 1) / G;
-  const int grid = kHeads * 8 * ((groups + 7) / 8);
-  hipLaunchKernelGGL(qkv_attention_kernel<BM>, dim3(grid), dim3(L::NT), L::LDS, s, X, Wp, fs, fc, cy,
-                     mask, ctx, batch, seq, G, c, eps);
+  const int grid = xcd_grid(groups, kHeads);
+  hipLaunchKernelGGL((qkv_attention_kernel<BM, WN, R, NP>), dim3(grid), dim3(L::NT), L::LDS, s, X,
+                     Wp, fs, fc, cy, mask, ctx, batch, seq, G, c, eps);
   return hipGetLastError();
+}
+
+// Rows of a workgroup (whole sentences).  Alone, where one workgroup per CU
+// covers the batch: the smallest of 64 / 128 / 192 / 256 rows that gives at
+// most kCus workgroups, with rings 3-4 slices deep (128 and 192 rows: negative,
+// their one-per-CU form).  Past that two workgroups a CU with rings of two
+// slices, 128 or 192 rows, whichever takes fewer rounds times rows.  Beside
+// other forwards (shared) always the latter, 192 rows where 128 would leave
+// a quarter or more of the tile idle (seq 48, 80, 96): deep rings would hold
+// the LDS that the other forwards' workgroups need (four-slot pass 3.93 ms
+// against 4.08).
+// Back to back launches (batch x seq), against 128 / 192-row workgroups that
+// copied for themselves: 1 x 16 7.4 -> 5.2 us, 64 x 16 8.5 -> 6.2, 64 x 32
+// 9.0 -> 7.1, 64 x 48 10.1 -> 8.8, 64 x 64 10.8 -> 9.4, 100 x 48 14.1 -> 10.2,
+// 32 x 128 11.7 -> 10.3; two a CU: 64 x 80 14.4 -> 12.9, 64 x 128 20.8 -> 18.1,
+// 500 x 16 17.2 -> 12.7.
+int qkv_attention_rows(int batch, int seq, bool shared) {
+  if (shared) return seq == 48 || seq == 80 || seq == 96 ? 192 : 128;
+  auto groups = [&](int rows) { return (batch + rows / seq - 1) / (rows / seq); };
+  for (int rows : {64, 128, 192, 256})
+    if (rows >= seq && kHeads * groups(rows) <= kCus) return rows == 128 || rows == 192 ? -rows : rows;
+  auto cost = [&](int rows) { return (kHeads * groups(rows) + 2 * kCus - 1) / (2 * kCus) * rows; };
+  return cost(128) < cost(192) ? 128 : 192;
 }
 
 bool qkv_attention_ok(int batch, int seq) {
@@ -1965,14 +1988,22 @@ bool qkv_attention_ok(int batch, int seq) {
 
 hipError_t qkv_attention(const f16* X, const f16* Wp, const float* fs, const float* fc,
                          const LnCarry& cy, const int32_t* mask, f16* ctx, int batch, int seq,
-                         float scale, float eps, hipStream_t s) {
+                         float scale, float eps, hipStream_t s, bool shared) {
   const bool aligned = (((uintptr_t)X | (uintptr_t)Wp | (uintptr_t)ctx) & 15) == 0 &&
                        (((uintptr_t)cy.st_in) & 15) == 0;
   if (!qkv_attention_ok(batch, seq) || !fc || !mask || !aligned) return hipErrorInvalidValue;
   const float c = scale * 1.4426950408889634f;  // scores * c are base-2 exponents
-  return qa::rows_for(seq) == 192
-             ? launch_qkv_attention<192>(X, Wp, fs, fc, cy, mask, ctx, batch, seq, c, eps, s)
-             : launch_qkv_attention<128>(X, Wp, fs, fc, cy, mask, ctx, batch, seq, c, eps, s);
+#define BBH_QA(...) \
+  launch_qkv_attention<__VA_ARGS__>(X, Wp, fs, fc, cy, mask, ctx, batch, seq, c, eps, s)
+  switch (qkv_attention_rows(batch, seq, shared)) {
+    case 64: return BBH_QA(64, 3, 4, 2);
+    case -128: return BBH_QA(128, 3, 3, 4);
+    case -192: return BBH_QA(192, 1, 3, 4);
+    case 256: return BBH_QA(256, 1, 3, 4);
+    case 192: return BBH_QA(192, 1, 2, 2);
+    default: return BBH_QA(128, 1, 2, 2);
+  }
+#undef BBH_QA
 }
 
 hipError_t gemm_fold(const f16* A, const f16* W, const LnCarry& cy, f16* C, int M, int N, int K,

@@ -67,7 +67,7 @@ hipError_t gemm_residual_stats(const f16* A, const f16* W, const f16* bias, cons
 bool qkv_attention_ok(int batch, int seq);
 hipError_t qkv_attention(const f16* X, const f16* Wp, const float* fs, const float* fc,
                          const LnCarry& cy, const int32_t* mask, f16* ctx, int batch, int seq,
-                         float scale, float eps, hipStream_t s);
+                         float scale, float eps, hipStream_t s, bool shared = false);
 
 // Tile configuration gemm() / gemm_residual_ln() launch for a shape (-1: the
 // plain tiled kernel), whether the LayerNorm is inside the GEMM kernel, and

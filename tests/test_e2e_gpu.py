@@ -352,6 +352,46 @@ def test_qkv_attention_kernel_equals_two_kernels(torch_cuda, ws, model):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("B,S", [
+    # One workgroup per CU, 64 rows: the last batch sizes before the next shape
+    # (21 groups), a sentence per group, and sentences that fill it unevenly.
+    (13, 16), (84, 16), (42, 32), (21, 48), (21, 64),
+    # 128, 192 and 256 rows, each just past the shape before
+    (85, 16), (43, 32), (22, 64), (21, 128), (63, 48), (43, 80), (84, 48), (85, 48), (63, 80),
+    (42, 112),
+    # two workgroups a CU: 128 rows, 192 rows
+    (64, 128), (43, 112), (500, 16), (512, 16), (64, 96), (170, 48), (127, 64)])
+def test_qkv_attention_workgroup_shapes(torch_cuda, ws, model, B, S):
+    # The workgroup shape follows from the batch, and from whether other
+    # forwards share the GPU (a pool of two slots); the bits do not.
+    from bbh import engine
+
+    torch = torch_cuda
+    rng = np.random.default_rng(B * S)
+    n = rng.integers(0, S + 1, size=B)
+    n[-1] = S
+    mask = (np.arange(S)[None, :] < n[:, None]).astype(np.int32)
+    mask[B // 2] = rng.integers(0, 2, S)  # keys masked anywhere
+    ids = rng.integers(1000, 30522, size=(B, S)).astype(np.int32)
+    types = rng.integers(0, 2, size=(B, S)).astype(np.int32)
+    want = _embed(torch, ws, model, ids, types, mask)
+    pool = engine.Pool(2, B, S)
+    got = _np(engine.embed_each(pool, model, engine.PackedBatches([(ids, types, mask)])))
+    # two segments of different lengths in one forward: the QKV GEMM and
+    # attention_kernel
+    extra = [np.ones((1, 16), np.int32) * k for k in (5, 0, 1)]
+    one = engine.Pool(1, B + 1, S)
+    two = _np(engine.embed_batches(one, model, engine.PackedBatches([(ids, types, mask), extra])))
+    torch.cuda.synchronize()
+    pool.close()
+    one.close()
+    assert np.array_equal(got, want)
+    if S != 16 and B * S + 16 <= 8192:
+        assert np.array_equal(two[:B], want)
+    else:  # one run, or past the carried LayerNorms: close only
+        assert np.abs(two[:B] - want).max() <= 2e-3
+
+
 @pytest.mark.parametrize("max_batch", [256, 1024])
 def test_pool_merges_equal_seq_batches(torch_cuda, ws, model, max_batch):
     # Length-grouped packing: each run of equal-seq batches executes as one
