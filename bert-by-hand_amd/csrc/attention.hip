@@ -36,8 +36,8 @@
 // Short sequences are bound by the global round trip: all of a workgroup's
 // loads (Q, K, V, mask) are issued before its single barrier, and the output
 // goes out through LDS as 16-byte stores of 64 contiguous bytes per row.
-// Long sequences are bound by exp + MFMA issue: a wavefront then takes two
-// query tiles at once, sharing each K and V^T operand read between them.
+// Long sequences are bound by exp + MFMA issue; at 16 tiles a wavefront takes
+// two query tiles at once, sharing each K and V^T operand read between them.
 
 #include <algorithm>
 
@@ -82,7 +82,7 @@ constexpr float kLazy = 8.f;
 // VL: packed sentences (sents[b] gives the rows and length; every token is
 // valid, `mask` and `seq` are unused).
 template <int NW, int T, int F, bool VL = false>
-__global__ __launch_bounds__(64 * NW, T == 2 ? 4 : 6) void attention_kernel(
+__global__ __launch_bounds__(64 * NW, T == 2 || NW > 8 ? 4 : 6) void attention_kernel(
     const f16* __restrict__ qkv, const int32_t* __restrict__ mask, f16* __restrict__ out,
     int batch, int seq, int heads, float c, const PackedSentence* __restrict__ sents) {
   HIP_DYNAMIC_SHARED(f16, smem);
@@ -204,7 +204,6 @@ __global__ __launch_bounds__(64 * NW, T == 2 ? 4 : 6) void attention_kernel(
         }
       }
       float mx[T];
-      bool up = false;
 #pragma unroll
       for (int t = 0; t < T; ++t) {
         // IEEE maximum (v_maximum3_f32): scores hold no NaN, and unlike fmaxf
@@ -219,21 +218,21 @@ __global__ __launch_bounds__(64 * NW, T == 2 ? 4 : 6) void attention_kernel(
                                                          false, false);
         mx[t] = __builtin_elementwise_maximum(__uint_as_float(sw[0]),
                                               __uint_as_float(sw[1]));  // finite: a key is unmasked
-        up = up || mx[t] > m[t] + lag;
       }
       if (!started) {
 #pragma unroll
         for (int t = 0; t < T; ++t) m[t] = mx[t];
         started = true;
-      } else if (__ballot(up)) {
+      } else {  // each tile for itself, so its bits do not depend on T
 #pragma unroll
-        for (int t = 0; t < T; ++t) {
-          const float mn = fmaxf(m[t], mx[t]);
-          const float corr = __builtin_amdgcn_exp2f((m[t] - mn) * c);
-          l[t] *= corr;
-          o[t] *= corr;
-          m[t] = mn;
-        }
+        for (int t = 0; t < T; ++t)
+          if (__ballot(mx[t] > m[t] + lag)) {
+            const float mn = fmaxf(m[t], mx[t]);
+            const float corr = __builtin_amdgcn_exp2f((m[t] - mn) * c);
+            l[t] *= corr;
+            o[t] *= corr;
+            m[t] = mn;
+          }
       }
       const f16* vrow = Vt + r32 * VLD + kc * 32 + 8 * kh;
       const f16x8 va = *reinterpret_cast<const f16x8*>(vrow);
@@ -330,13 +329,17 @@ hipError_t launch_attention(const f16* qkv, const int32_t* mask, f16* merged, in
   return hipGetLastError();
 }
 
-// Workgroup shape by query-tile count (tiles = ceil(seq / 32)).  Up to 7
-// tiles: one tile per wavefront, output staged through the K/V area.  8 tiles:
-// 4 wavefronts x 2 tiles.  16 tiles: 8 x 2, output staged through the K/V
-// area too (16-byte stores of 64-byte row runs; 2% faster at batch 256 x 512
-// than the 8-byte stores from the accumulator layout).  9-15: 8 x 1 (a 2-tile
-// grouping would leave wavefronts computing empty tiles).  For packed
-// sentences the longest one sets the shape.
+// Workgroup shape by query-tile count (tiles = ceil(seq / 32)).  Up to 4
+// tiles: one tile per wavefront, output staged through the K/V area.  5-8: 8
+// wavefronts, 9-15: 12, one tile at a time and stored straight from the
+// accumulators: more wavefronts than tiles still help to stage K and V, and
+// more of them hide the exp and MFMA latencies than 4 or 8, or two tiles a
+// wavefront (64 x 144 / 160 / 192 / 224 / 256 11.2 / 11.0 / 13.7 / 16.8 / 19.5
+// -> 9.0 / 9.5 / 12.5 / 15.3 / 18.6 us, 21 x 304 12.5 -> 11.3, 40 x 320 / 384 /
+// 448 19.1 / 22.6 / 31.5 -> 17.9 / 22.1 / 29.8).  16: 8 x 2, each operand read
+// serving two tiles, output staged through the K/V area (256 x 512: 172 us
+// against 174 for 12 x 1 and 182 for 8 x 1).  For packed sentences the longest
+// one sets the shape.
 template <bool VL>
 hipError_t attention_any(const f16* qkv, const int32_t* mask, f16* merged, int batch, int heads,
                          int seq, float scale, hipStream_t s, const PackedSentence* sents) {
@@ -345,9 +348,9 @@ hipError_t attention_any(const f16* qkv, const int32_t* mask, f16* merged, int b
 #define BBH_ATT(NW, T, F) \
   launch_attention<NW, T, F, VL>(qkv, mask, merged, batch, heads, seq, c, s, sents)
   if (tiles >= 16) return BBH_ATT(8, 2, 3);
-  if (tiles > 8) return BBH_ATT(8, 1, 0);
-  if (tiles == 8) return BBH_ATT(4, 2, 3);
-  if (tiles >= 4) return BBH_ATT(4, 1, 3);
+  if (tiles > 8) return BBH_ATT(12, 1, 0);
+  if (tiles > 4) return BBH_ATT(8, 1, 0);
+  if (tiles == 4) return BBH_ATT(4, 1, 3);
   if (tiles >= 2) return BBH_ATT(2, 1, 3);
   return BBH_ATT(1, 1, 3);
 #undef BBH_ATT

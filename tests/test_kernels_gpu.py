@@ -318,6 +318,34 @@ def test_fused_attention(torch_cuda, S, kind):
         assert np.all(got[S:2 * S] == 0.0)
 
 
+def test_attention_bits_do_not_depend_on_the_padding(torch_cuda):
+    # Every workgroup shape (1 to 16 query tiles) takes the same rescale
+    # decisions per tile and the same key order: a sentence's rows are, bit for
+    # bit, the same at every padded length, scores rising along the keys
+    # included.
+    torch = torch_cuda
+    from bbh import engine
+
+    rng = np.random.default_rng(7)
+    for n in (16, 45, 100, 130, 250, 300):
+        qkv = _h(rng, (2, 512, 1152), 2.0)
+        qkv[0, :, 384:768] += (np.arange(512)[:, None] * 0.02).astype(np.float16)
+        ref = None
+        for S in sorted({-(-n // 16) * 16} | {x for x in (64, 112, 128, 144, 176, 208, 256, 288, 400, 496, 512)
+                                              if x >= n}):
+            mask = np.zeros((2, S), np.int32)
+            mask[:, :n] = 1
+            out = torch.empty((2 * S, 384), dtype=torch.float16, device="cuda")
+            x = to_dev(torch, qkv[:, :S].reshape(2 * S, 1152))
+            engine.launch_attention(x, to_dev(torch, mask), out, 2, S)
+            got = out.cpu().numpy().reshape(2, S, 384)[:, :n]
+            ref = got if ref is None else ref
+            # rows of a part-filled 32-query tile share its rescale decisions
+            # with the rows past the sentence: compare whole tiles
+            assert np.array_equal(got[:, :n // 32 * 32], ref[:, :n // 32 * 32]), (n, S)
+            assert np.abs(got.astype(np.float32) - ref.astype(np.float32)).max() <= 4e-3, (n, S)
+
+
 def test_unfused_attention_pieces_match_fused(torch_cuda):
     # launch_attention_scores -> launch_softmax(mask) -> launch_attention_context
     # (src/model/encoder.cu:39-45) against the oracle and the fused kernel.
