@@ -269,9 +269,9 @@ def kernel_name(engine, op, tile, fused, batch=0, seq=0):
 
 
 def gemm_grid_items(tile_name, M, N):
-    """Work-items of a tiled-GEMM launch (the launcher's grid: the tiles dealt to
-    8 XCDs, or to one XCD a row of tiles below 8 rows of at most 32 tiles;
-    64 threads for each computing and each copying wavefront), as rocprofv3
+    """Work-items of a tiled-GEMM launch (the launcher's grid: whole rows of tiles
+    dealt to 8 XCDs from 96 rows on, below that the tiles in even spans, below 8
+    rows of at most 32 tiles one XCD a row; 64 threads for each computing and each copying wavefront), as rocprofv3
     reports Grid_Size; None for other kernels."""
     import re
 
@@ -281,7 +281,8 @@ def gemm_grid_items(tile_name, M, N):
     bm, bn, wm, wn, _, pd = (int(x) for x in m.groups())
     rows, cols = -(-M // bm), N // bn
     xcds = rows if rows < 8 and cols <= 32 else 8
-    return -(-rows * cols // xcds) * 8 * 64 * (wm * wn + (-pd // 16 if pd < 0 else 0))
+    per_xcd = -(-rows // 8) * cols if rows >= 96 else -(-rows * cols // xcds)
+    return per_xcd * 8 * 64 * (wm * wn + (-pd % 256 // 16 if pd < 0 else 0))
 
 
 def classify(engine, recs, steps):

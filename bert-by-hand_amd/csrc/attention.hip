@@ -88,10 +88,13 @@ __global__ __launch_bounds__(64 * NW, T == 2 || NW > 8 ? 4 : 6) void attention_k
   HIP_DYNAMIC_SHARED(f16, smem);
   // (sequence, head) of this workgroup; the heads of a sequence go to one XCD
   // back to back (but where its span ends), so its QKV rows are fetched into
-  // one L2.
+  // one L2.  Last sequence first: the QKV Linear wrote its rows in ascending
+  // order, and of more than the 256 MB that the memory-side cache holds (302 MB
+  // at 256 x 512) the last ones are still there, where an ascending walk would
+  // evict each row before it is read (bert_embed 256 x 512 4.46 -> 4.37 ms).
   const int item = xcd_item(batch, heads);
   if (item < 0) return;
-  const int b = item / heads, h = item - b * heads;
+  const int bq = item / heads, h = item - bq * heads, b = batch - 1 - bq;
   size_t row0 = (size_t)b * seq;  // first hidden row of the sentence
   if constexpr (VL) {
     const PackedSentence sn = sents[b];
@@ -305,9 +308,9 @@ __global__ __launch_bounds__(64 * NW, T == 2 || NW > 8 ? 4 : 6) void attention_k
         }
     }
   }
-  // A packed sentence may have fewer query tiles than the workgroup has
-  // wavefronts; those wavefronts still take part in the staging barrier.
-  if constexpr (VL && (F & 2)) {
+  // A sentence may have fewer query tiles than the workgroup has wavefronts;
+  // those wavefronts still take part in the staging barrier.
+  if constexpr (F & 2) {
     if (NW > 1 && nch <= NW * T && wave >= nch) __syncthreads();
   }
 }
@@ -329,17 +332,19 @@ hipError_t launch_attention(const f16* qkv, const int32_t* mask, f16* merged, in
   return hipGetLastError();
 }
 
-// Workgroup shape by query-tile count (tiles = ceil(seq / 32)).  Up to 4
-// tiles: one tile per wavefront, output staged through the K/V area.  5-8: 8
-// wavefronts, 9-15: 12, one tile at a time and stored straight from the
-// accumulators: more wavefronts than tiles still help to stage K and V, and
-// more of them hide the exp and MFMA latencies than 4 or 8, or two tiles a
-// wavefront (64 x 144 / 160 / 192 / 224 / 256 11.2 / 11.0 / 13.7 / 16.8 / 19.5
-// -> 9.0 / 9.5 / 12.5 / 15.3 / 18.6 us, 21 x 304 12.5 -> 11.3, 40 x 320 / 384 /
-// 448 19.1 / 22.6 / 31.5 -> 17.9 / 22.1 / 29.8).  16: 8 x 2, each operand read
-// serving two tiles, output staged through the K/V area (256 x 512: 172 us
-// against 174 for 12 x 1 and 182 for 8 x 1).  For packed sentences the longest
-// one sets the shape.
+// Workgroup shape by query-tile count (tiles = ceil(seq / 32); for packed
+// sentences of the longest one).  2-4 tiles: 4 wavefronts of one tile each,
+// output staged through the K/V area.  5-8: 8 wavefronts, 9-16: 12, one tile at
+// a time and stored straight from the accumulators: more wavefronts than
+// tiles still help to stage K and V, and more of them hide the exp and MFMA
+// latencies than 4 or 8, or two tiles a wavefront (266 x 96 21.2 -> 17.6 us, 600
+// x 64 23.6 -> 22.1, 64 x 144 / 192 / 256 11.2 / 13.7 / 19.5 -> 9.0 / 12.5 /
+// 18.6, 21 x 304 12.5 -> 11.3, 80 x 288 / 480 28.0 / 54.9 -> 27.1 / 52.3, 128 x
+// 512 85.6 -> 81.2).  Where a CU's share of workgroups fills it anyway: 9-11
+// tiles on 8 wavefronts (three workgroups a CU against two: 160 x 288 47.2 ->
+// 44.9), 16 on 8 x 2, each operand read serving two tiles, output staged (256
+// x 512 174 -> 172).  Packed sentences of up to 3 tiles: 2 wavefronts, for most
+// sentences are much shorter than the longest.
 template <bool VL>
 hipError_t attention_any(const f16* qkv, const int32_t* mask, f16* merged, int batch, int heads,
                          int seq, float scale, hipStream_t s, const PackedSentence* sents) {
@@ -347,11 +352,14 @@ hipError_t attention_any(const f16* qkv, const int32_t* mask, f16* merged, int b
   const int tiles = (seq + 31) / 32;
 #define BBH_ATT(NW, T, F) \
   launch_attention<NW, T, F, VL>(qkv, mask, merged, batch, heads, seq, c, s, sents)
-  if (tiles >= 16) return BBH_ATT(8, 2, 3);
-  if (tiles > 8) return BBH_ATT(12, 1, 0);
+  const int wgs = batch * heads;
+  if (tiles >= 16 && wgs > 2048) return BBH_ATT(8, 2, 3);
+  if (tiles > (wgs > 1280 ? 11 : 8)) return BBH_ATT(12, 1, 0);
   if (tiles > 4) return BBH_ATT(8, 1, 0);
-  if (tiles == 4) return BBH_ATT(4, 1, 3);
-  if (tiles >= 2) return BBH_ATT(2, 1, 3);
+  if (tiles >= (VL ? 4 : 2)) return BBH_ATT(4, 1, 3);
+  if constexpr (VL) {
+    if (tiles >= 2) return BBH_ATT(2, 1, 3);
+  }
   return BBH_ATT(1, 1, 3);
 #undef BBH_ATT
 }

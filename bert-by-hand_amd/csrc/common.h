@@ -25,24 +25,35 @@ constexpr size_t kLdsMax = 160 * 1024;  // LDS per workgroup on gfx950
 constexpr int kTypes = 2;
 
 // Workgroup b runs on XCD b % 8, each XCD with its own L2 and 32 CUs.
-// xcd_item deals rows * cols items (row-major) to the XCDs in contiguous spans
-// whose lengths differ by at most one, and gives this workgroup's item, or
-// -1: the items of a row share operands, so they share an L2, the same rows
-// stay on the same XCD from kernel to kernel, and no XCD gets more than its
-// eighth.  Fewer than 8 rows of at most 32 items keep to one XCD each (the
-// next kernel finds them in that L2: FFN1 at 16 rows 3.8 us inside a forward
-// against 4.4 over all XCDs).  The grid is xcd_grid(rows, cols) workgroups.
-constexpr int kXcds = 8, kXcdCus = 32;
+// xcd_item deals rows * cols items (row-major) to the XCDs and gives this
+// workgroup's item, or -1.  The items of a row share operands, so they go to
+// one XCD's L2.
+//  - From kXcdRows rows on, row r goes to XCD r % 8, in order (spans, below,
+//    measured slower there: FFN2 at 46656 rows 97 us against 89).
+//  - Below that, contiguous spans whose lengths differ by at most one item: no
+//    XCD gets more than its eighth (50 whole rows would be 7 on two XCDs and 6
+//    on the others), and the same rows stay on the same XCD from kernel to
+//    kernel.
+//  - Fewer than 8 rows of at most 32 items keep to one XCD each (the next
+//    kernel finds them in that L2: FFN1 at 16 rows 3.8 us inside a forward
+//    against 4.4 over all XCDs).
+// The grid is xcd_grid(rows, cols) workgroups.
+constexpr int kXcds = 8, kXcdCus = 32, kXcdRows = 96;
 __host__ __device__ inline int xcds_for(int rows, int cols) {
   return rows < kXcds && cols <= kXcdCus ? rows : kXcds;
 }
 __host__ __device__ inline int xcd_grid(int rows, int cols) {
+  if (rows >= kXcdRows) return (rows + kXcds - 1) / kXcds * cols * kXcds;
   const int n = xcds_for(rows, cols);
   return (rows * cols + n - 1) / n * kXcds;
 }
 __device__ __forceinline__ int xcd_item(int rows, int cols) {
-  const int n = xcds_for(rows, cols), q = rows * cols / n, r = rows * cols % n;
   const int x = blockIdx.x % kXcds, k = blockIdx.x / kXcds;
+  if (rows >= kXcdRows) {
+    const int row = k / cols * kXcds + x;
+    return row < rows ? row * cols + k % cols : -1;
+  }
+  const int n = xcds_for(rows, cols), q = rows * cols / n, r = rows * cols % n;
   return x < n && k < q + (x < r ? 1 : 0) ? x * q + min(x, r) + k : -1;
 }
 

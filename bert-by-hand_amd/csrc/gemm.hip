@@ -47,20 +47,21 @@ enum Epi { kBias = 0, kGelu = 1, kResidual = 2, kLayerNorm = 3, kFold = 4, kFold
 
 template <int BM_, int BN_, int WM_, int WN_, int SA_, int PD_ = 0, int SW_ = 2>
 struct Cfg {
-  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, SA = SA_, SW = SW_, BK = 64;
+  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, SA = SA_, SW = SW_;
   // PD_ > 0: register prefetch depth (mainloop_reg).  PD_ = -(16 NP + KPB):
   // one ring of whole slices (mainloop_deep), KPB of them per barrier, copied
   // by NP wavefronts of their own beside the WM x WN that compute (NP = 0: by
-  // those).
+  // those); 256 more: slices 32 wide instead of 64.
   static constexpr int PD = PD_ > 0 ? PD_ : 0;
-  static constexpr int KPB = PD_ < 0 ? -PD_ % 16 : 1, NP = PD_ < 0 ? -PD_ / 16 : 0;
-  using L = Slice<64>;
+  static constexpr int KPB = PD_ < 0 ? -PD_ % 16 : 1, NP = PD_ < 0 ? -PD_ / 16 % 16 : 0;
+  static constexpr int BK = -PD_ >= 256 ? 32 : 64, RPC = 512 / BK;  // rows of a 1 KB copy
+  using L = Slice<BK>;
   static constexpr int NW = WM * WN, THREADS = 64 * (NW + NP);
   static constexpr int NC = NP > 0 ? NP : NW;            // wavefronts that issue the copies
   static constexpr bool DEEP = PD_ < 0;
   static constexpr int TM = BM / WM, TN = BN / WN;  // wave tile
   static constexpr int FM = TM / 32, FN = TN / 32;  // 32x32 blocks per wave
-  static constexpr int LA = BM / (8 * NC), LW = BN / (8 * NC);  // copies per thread per slice
+  static constexpr int LA = BM / (RPC * NC), LW = BN / (RPC * NC);  // copies per thread per slice
   static constexpr int A_STAGE = BM * BK, W_STAGE = BN * BK;  // halves per slice
   static constexpr int W_BASE = SA * A_STAGE;                 // W ring follows the A ring
   static constexpr int OUT_LD = BN + 8;                       // padded row of the fp16 output tile
@@ -75,7 +76,7 @@ struct Cfg {
   static constexpr size_t LDS = RING > OUT ? RING : OUT;
   static_assert(NW + NP <= 16, "wavefronts");
   static_assert(TM % 32 == 0 && TN % 32 == 0, "wave tile is whole 32x32 blocks");
-  static_assert(BM % (8 * NC) == 0 && BN % (8 * NC) == 0, "load distribution");
+  static_assert(BM % (RPC * NC) == 0 && BN % (RPC * NC) == 0, "load distribution");
   static_assert(SA >= 2 && SW >= 2, "ring depths");
   static_assert(!DEEP || (SA == SW && SA % KPB == 0 && SA >= 2 * KPB), "one ring of whole groups");
   // vmcnt that may stay outstanding when slice kt must have landed: the
@@ -88,8 +89,8 @@ struct Cfg {
 };
 
 // Copying one 64-wide K slice of ROWS K-contiguous rows into LDS: each
-// wavefront instruction fills 1 KB = 8 rows; lane i lands at row i / 8, slot
-// i % 8 of them, so it fetches the logical chunk that belongs in that slot.
+// wavefront instruction fills 1 KB = 8 rows (16 of a 32-wide slice); lane i
+// lands at row i / 8, slot i % 8 of them, so it fetches the logical chunk that belongs in that slot.
 // Rows at or past `valid` are read clamped to row valid-1.  row_offsets gives
 // off[j] = byte offset of this lane's chunk of copy j from the slice base,
 // computed once per tile; issue_rows_at then copies a slice through a buffer
@@ -100,28 +101,30 @@ struct Cfg {
 __device__ __forceinline__ int wave_id() {
   return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 }
-template <int ROWS, int NW>
-__device__ __forceinline__ void row_offsets(int ld, int valid, uint32_t (&off)[ROWS / (8 * NW)],
+template <int ROWS, int NW, int BK = 64>
+__device__ __forceinline__ void row_offsets(int ld, int valid,
+                                            uint32_t (&off)[ROWS * BK / (512 * NW)],
                                             int wave = wave_id()) {
+  constexpr int n = ROWS * BK / (512 * NW), CPR = BK / 8;  // copies; 16-byte chunks a row
   const int lane = threadIdx.x & 63;
 #pragma unroll
-  for (int j = 0; j < ROWS / (8 * NW); ++j) {
-    const int r = (wave * (ROWS / (8 * NW)) + j) * 8 + (lane >> 3);
-    off[j] = (uint32_t)(min(r, valid - 1) * ld + (((lane & 7) ^ Slice<64>::f(r)) << 3)) * 2u;
+  for (int j = 0; j < n; ++j) {
+    const int r = (wave * n + j) * (512 / BK) + lane / CPR;
+    off[j] = (uint32_t)(min(r, valid - 1) * ld + (((lane % CPR) ^ Slice<BK>::f(r)) << 3)) * 2u;
   }
 }
 
 // One slice's copies: lane chunk offsets from row_offsets, slice offset
 // `soff` bytes (wave-uniform).
-template <int ROWS, int NW>
+template <int N>
 __device__ __forceinline__ void issue_rows_at(__amdgpu_buffer_rsrc_t src, uint32_t soff,
-                                              const uint32_t (&off)[ROWS / (8 * NW)], f16* buf,
+                                              const uint32_t (&off)[N], f16* buf,
                                               int wave = wave_id()) {
 #pragma unroll
-  for (int j = 0; j < ROWS / (8 * NW); ++j)
+  for (int j = 0; j < N; ++j)
     __builtin_amdgcn_raw_ptr_buffer_load_lds(
-        src, (__attribute__((address_space(3))) void*)(buf + (wave * (ROWS / (8 * NW)) + j) * 8 * 64),
-        16, (int)off[j], (int)soff, 0, 0);
+        src, (__attribute__((address_space(3))) void*)(buf + (wave * N + j) * 512), 16, (int)off[j],
+        (int)soff, 0, 0);
 }
 
 // Scheduling groups: (one DS read, then ~Q/R MFMAs) x R.
@@ -212,10 +215,10 @@ __device__ __forceinline__ void mainloop(const f16* __restrict__ A, const f16* _
   const __amdgpu_buffer_rsrc_t rA = buffer_of(a0, (uint32_t)(M - m0) * K * 2u);
   const __amdgpu_buffer_rsrc_t rW = buffer_of(w0, (uint32_t)C::BN * K * 2u);
   auto issueA = [&](int s) {
-    issue_rows_at<C::BM, C::NW>(rA, s * C::BK * 2, offA, ringA + (s % C::SA) * C::A_STAGE);
+    issue_rows_at(rA, s * C::BK * 2, offA, ringA + (s % C::SA) * C::A_STAGE);
   };
   auto issueW = [&](int s) {
-    issue_rows_at<C::BN, C::NW>(rW, s * C::BK * 2, offW, ringW + (s % C::SW) * C::W_STAGE);
+    issue_rows_at(rW, s * C::BK * 2, offW, ringW + (s % C::SW) * C::W_STAGE);
   };
   // Slice s of W is issued SW-1 iterations and slice s of A SA-1 iterations
   // before it is consumed; the prologue is iterations j = 1-max(SA,SW) .. -1
@@ -320,8 +323,8 @@ __device__ __forceinline__ void mainloop_deep(const f16* __restrict__ A,
   const __amdgpu_buffer_rsrc_t rA = buffer_of(A + (size_t)m0 * K, (uint32_t)(M - m0) * K * 2u);
   const __amdgpu_buffer_rsrc_t rW = buffer_of(W + (size_t)n0 * K, (uint32_t)C::BN * K * 2u);
   auto issue = [&](int s, int slot) {
-    issue_rows_at<C::BN, C::NC>(rW, s * C::BK * 2, offW, ringW + slot * C::W_STAGE, cw);
-    issue_rows_at<C::BM, C::NC>(rA, s * C::BK * 2, offA, ringA + slot * C::A_STAGE, cw);
+    issue_rows_at(rW, s * C::BK * 2, offW, ringW + slot * C::W_STAGE, cw);
+    issue_rows_at(rA, s * C::BK * 2, offA, ringA + slot * C::A_STAGE, cw);
   };
   int slot = 0;  // of slice kt
   // Slices kt .. kt+P-1 landed: the copies of newer groups may be in flight (a
@@ -336,8 +339,8 @@ __device__ __forceinline__ void mainloop_deep(const f16* __restrict__ A,
       if (kt + R - P + d < KT) issue(kt + R - P + d, (slot + R - P + d) % R);
   };
   if (copies) {
-    row_offsets<C::BM, C::NC>(K, M - m0, offA, cw);
-    row_offsets<C::BN, C::NC>(K, C::BN, offW, cw);
+    row_offsets<C::BM, C::NC, C::BK>(K, M - m0, offA, cw);
+    row_offsets<C::BN, C::NC, C::BK>(K, C::BN, offW, cw);
 #pragma unroll
     for (int d = 0; d < R - P; ++d)
       if (d < KT) issue(d, d);
@@ -620,6 +623,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave / C::WN, wn = wave % C::WN;
   const int r32 = lane & 31, kh = lane >> 5;
+  const bool computes = C::NP == 0 || wave < C::NW;  // else one of mainloop_deep's copying wavefronts
 
   // Per-column operands (bias; gamma and beta for LayerNorm) depend only on
   // the lane's columns.  Tiles with room in registers load them once, all
@@ -756,7 +760,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(
     }
     fcol = fc_lds;
     lds_barrier();
-    if (C::NP == 0 || wave < C::NW) {
+    if (computes) {
 #pragma unroll
       for (int fm = 0; fm < C::FM; ++fm) {
         const int row = wm * C::TM + fm * 32 + r32;
@@ -767,7 +771,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(
   }
 
   if constexpr (EPI == kLayerNorm) {
-    static_assert(C::BN == kHidden && C::NP == 0, "LayerNorm tile owns whole 384-wide rows");
+    static_assert(C::BN == kHidden, "LayerNorm tile owns whole 384-wide rows");
     // v = acc + bias + residual, then the row statistics (lane ^ 32 holds the
     // other half of the wave's columns, LDS across wn).
     // The residual rows arrive through the (still free) output staging area:
@@ -777,16 +781,17 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(
     // accumulators are live), unpadded [BM][384] with LDS chunk slot c of
     // row r holding logical chunk (c & ~7) | ((c ^ r) & 7).
     constexpr bool kStageRes = C::NPASS == 1;
-    constexpr int kResCopies = C::BM * (kHidden / 8) / 64;  // 1 KB copies
-    static_assert(!kStageRes || kResCopies % C::NW == 0, "residual copies per wavefront");
+    constexpr int kResCopies = C::BM * (kHidden / 8) / 64;  // 1 KB copies, by all wavefronts
+    constexpr int kAll = C::NW + C::NP;
     auto res_at = [&](int r, int n) {  // halves offset of column n of staged row r
       const int c = n >> 3;
       return r * kHidden + (((c & ~7) | ((c ^ r) & 7)) << 3) + (n & 7);
     };
     if constexpr (kStageRes) {
 #pragma unroll
-      for (int j = 0; j < kResCopies / C::NW; ++j) {
-        const int g = j * C::NW + wave;  // 1 KB copy index
+      for (int j = 0; j < (kResCopies + kAll - 1) / kAll; ++j) {
+        const int g = j * kAll + wave_id();  // 1 KB copy index
+        if (kResCopies % kAll != 0 && g >= kResCopies) break;
         const int q = g * 64 + lane, r = q / (kHidden / 8), c = q % (kHidden / 8);
         const int cl = (c & ~7) | ((c ^ r) & 7);
         __builtin_amdgcn_global_load_lds(residual + (size_t)min(m0 + r, M - 1) * kHidden + cl * 8,
@@ -796,22 +801,24 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(
       wait_vm<0>();
       lds_barrier();
     }
+    if (computes) {
 #pragma unroll
-    for (int fn = 0; fn < C::FN; ++fn) {
-      if constexpr (!kHoist) load_cols(fn, 0);
-      const int h = kHoist ? fn : 0;
+      for (int fn = 0; fn < C::FN; ++fn) {
+        if constexpr (!kHoist) load_cols(fn, 0);
+        const int h = kHoist ? fn : 0;
 #pragma unroll
-      for (int fm = 0; fm < C::FM; ++fm) {
-        const int ml = wm * C::TM + fm * 32 + r32;
-        const int mg = min(m0 + ml, M - 1);
+        for (int fm = 0; fm < C::FM; ++fm) {
+          const int ml = wm * C::TM + fm * 32 + r32;
+          const int mg = min(m0 + ml, M - 1);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int n = wn * C::TN + fn * 32 + 8 * j + 4 * kh;
-          const f16x4 rv =
-              kStageRes ? *reinterpret_cast<const f16x4*>(tile + res_at(ml, n))
-                        : *reinterpret_cast<const f16x4*>(residual + (size_t)mg * kHidden + n);
+          for (int j = 0; j < 4; ++j) {
+            const int n = wn * C::TN + fn * 32 + 8 * j + 4 * kh;
+            const f16x4 rv =
+                kStageRes ? *reinterpret_cast<const f16x4*>(tile + res_at(ml, n))
+                          : *reinterpret_cast<const f16x4*>(residual + (size_t)mg * kHidden + n);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[fm][fn][4 * j + i] += (float)bvs[h][j][i] + (float)rv[i];
+            for (int i = 0; i < 4; ++i) acc[fm][fn][4 * j + i] += (float)bvs[h][j][i] + (float)rv[i];
+          }
         }
       }
     }
@@ -819,42 +826,46 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(
     // deviation over its TN columns of the row, combined across the WN
     // wavefronts of the row as equal-size groups (Chan et al.).
     float2* red2 = reinterpret_cast<float2*>(red);  // [WN][BM]
+    if (computes) {
 #pragma unroll
-    for (int fm = 0; fm < C::FM; ++fm) {
-      float s = 0.f;
+      for (int fm = 0; fm < C::FM; ++fm) {
+        float s = 0.f;
 #pragma unroll
-      for (int fn = 0; fn < C::FN; ++fn)
+        for (int fn = 0; fn < C::FN; ++fn)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) s += acc[fm][fn][i];
-      const float mw = xor32_sum(s) * (1.0f / C::TN);
-      float q = 0.f;
+          for (int i = 0; i < 16; ++i) s += acc[fm][fn][i];
+        const float mw = xor32_sum(s) * (1.0f / C::TN);
+        float q = 0.f;
 #pragma unroll
-      for (int fn = 0; fn < C::FN; ++fn)
+        for (int fn = 0; fn < C::FN; ++fn)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const float d = acc[fm][fn][i] - mw;
-          q += d * d;
-        }
-      q = xor32_sum(q);
-      if (kh == 0) red2[wn * C::BM + wm * C::TM + fm * 32 + r32] = make_float2(mw, q);
+          for (int i = 0; i < 16; ++i) {
+            const float d = acc[fm][fn][i] - mw;
+            q += d * d;
+          }
+        q = xor32_sum(q);
+        if (kh == 0) red2[wn * C::BM + wm * C::TM + fm * 32 + r32] = make_float2(mw, q);
+      }
     }
     lds_barrier();
+    if (computes) {
 #pragma unroll
-    for (int fm = 0; fm < C::FM; ++fm) {
-      const int row = wm * C::TM + fm * 32 + r32;
-      float t = 0.f;
+      for (int fm = 0; fm < C::FM; ++fm) {
+        const int row = wm * C::TM + fm * 32 + r32;
+        float t = 0.f;
 #pragma unroll
-      for (int w = 0; w < C::WN; ++w) t += red2[w * C::BM + row].x;
-      mean[fm] = t * (1.0f / C::WN);
-      float t2 = 0.f, dd = 0.f;
+        for (int w = 0; w < C::WN; ++w) t += red2[w * C::BM + row].x;
+        mean[fm] = t * (1.0f / C::WN);
+        float t2 = 0.f, dd = 0.f;
 #pragma unroll
-      for (int w = 0; w < C::WN; ++w) {
-        const float2 pw = red2[w * C::BM + row];
-        const float d = pw.x - mean[fm];
-        t2 += pw.y;
-        dd += d * d;
+        for (int w = 0; w < C::WN; ++w) {
+          const float2 pw = red2[w * C::BM + row];
+          const float d = pw.x - mean[fm];
+          t2 += pw.y;
+          dd += d * d;
+        }
+        rstd[fm] = rsqrtf(fmaf((float)C::TN, dd, t2) * (1.0f / kHidden) + eps);
       }
-      rstd[fm] = rsqrtf(fmaf((float)C::TN, dd, t2) * (1.0f / kHidden) + eps);
     }
   }
 
@@ -866,7 +877,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(
   // fence keeps a single block's values live.
 #pragma unroll
   for (int p = 0; p < C::NPASS; ++p) {
-    if ((C::NPASS == 1 || wm == p) && (C::NP == 0 || wave < C::NW)) {
+    if ((C::NPASS == 1 || wm == p) && computes) {
 #pragma unroll
       for (int fn = 0; fn < C::FN; ++fn) {
         if constexpr (!kHoist) load_cols(fn, 0);
@@ -1543,12 +1554,13 @@ __global__ __launch_bounds__(wres::THREADS) void gemm_wres_kernel(
   }
 }
 
-// The weight-resident kernel serves K = 384 and N a multiple of 384, from
-// the M where sweeps on MI355X show it ahead of the tiled kernels: 16384 for
-// FFN1 (N = 1536, where it saves the most L2 traffic per row), 24576 for QKV.
-bool wres_ok(int M, int N, int K) {
-  return K == wres::K && N % wres::COLS == 0 && M >= (N >= 1536 ? 16384 : 24576);
-}
+// The weight-resident kernel serves K = 384 and N a multiple of 384 above the
+// rows of the carried LayerNorms, where its two passes over W per CU (the
+// prologue) are paid back.  Back to back launches against the tiles: FFN1 +
+// GELU at 8704 / 12288 / 15360 rows 23.7 / 29.2 / 34.4 -> 20.6 / 24.4 / 29.7
+// us; QKV at 10240 / 12288 / 15360 / 20480 rows 16.8 / 19.8 / 23.7 / 28.8 ->
+// 16.1 / 17.7 / 20.6 / 24.8 us.
+bool wres_ok(int M, int N, int K) { return K == wres::K && N % wres::COLS == 0 && M > 8192; }
 
 template <int EPI>
 hipError_t launch_wres(const f16* A, const f16* W, const f16* bias, f16* out, int M, int N,
@@ -1843,6 +1855,8 @@ int pick_plain(int M, int N, int K, bool shared) {
     id = qkv ? 30 : ffn1 ? (shared ? 26 : 19) : wide_k ? 31 : 0;
   else if (M <= 8192)
     id = shared ? (wide_k ? 31 : 30) : qkv || ffn1 ? 19 : wide_k ? 30 : 0;
+  else if (M <= 10880)
+    id = wide_k ? 40 : 30;
   else if (M <= 16384)
     id = wide_k ? 32 : 30;
   else if (M <= 49152)
@@ -1861,17 +1875,20 @@ int gemm_tile(int M, int N, int K, bool shared) {
   return wres_ok(M, N, K) ? kTiles : pick_plain(M, N, K, shared);
 }
 
-// Large M: one kernel whose 128x384 tile owns whole rows.  Smaller M: a tile
-// that owns whole rows leaves most CUs idle and streams all of W per
-// workgroup, so the GEMM runs on 2-D tiles with a bias + residual epilogue
-// (in place over y) and the row LayerNorm follows as its own pass.
-// The weight-resident kernel takes the K = 384 LayerNorm Linear (O-proj)
-// from M = 65536, where it passes tile 28 (89.5 vs 98.0 us at M = 131072;
-// at M = 26857 its fixed W prologue leaves it 15% behind).
+// Large M: one kernel that owns whole rows.  Smaller M: a tile that owns whole
+// rows leaves most CUs idle and streams all of W per workgroup, so the GEMM
+// runs on 2-D tiles with a bias + residual epilogue (in place over y) and the
+// row LayerNorm follows as its own pass.  K = 384 (O-proj): the
+// weight-resident kernel above the rows of the carried LayerNorms (8704 /
+// 15360 / 20480 / 65536 rows 12.1 / 13.1 / 16.9 / 37.6 us against 13.0 / 15.0 /
+// 19.3 / 46.3 for the best tile).  Wider K (FFN2): whole-row tiles once tile 40
+// needs a second round of workgroups (8704 / 10240 rows: 16.3 / 17.3 us and a
+// 5.5-6 us pass against 30.4 / 31.0 on 64x384; 15360: 27.6 and 7.5 against
+// 33.3).
 int gemm_residual_ln_tile(int M, int K, bool* fused_ln, bool shared) {
-  *fused_ln = M > 8192;
+  *fused_ln = K == wres::K ? M > 8192 : M > std::max(8192, kCus / 3 * 128);
   if (!*fused_ln) return pick_plain(M, kHidden, K, shared);
-  if (K == wres::K && M >= 65536) return kTiles;
+  if (K == wres::K) return kTiles;
   return M <= 16384 ? 14 : K >= 1024 ? 18 : 28;
 }
 

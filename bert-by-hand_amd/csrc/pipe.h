@@ -20,6 +20,14 @@ struct Slice<64> {
   __device__ static __forceinline__ int off(int r, int c) { return r * 64 + ((c ^ f(r)) << 3); }
 };
 
+// The same for a 32-wide K slice: 64 bytes = 4 chunks a row, f(r) = (r >> 2) & 3
+// (rows r and r + 4 share their 16 banks).
+template <>
+struct Slice<32> {
+  __device__ static __forceinline__ int f(int r) { return (r >> 2) & 3; }
+  __device__ static __forceinline__ int off(int r, int c) { return r * 32 + ((c ^ f(r)) << 3); }
+};
+
 // s_waitcnt vmcnt(n) with the other counters left alone (gfx9 encoding).
 template <int N>
 __device__ __forceinline__ void wait_vm() {
