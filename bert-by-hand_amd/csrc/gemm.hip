@@ -1881,12 +1881,12 @@ int gemm_tile(int M, int N, int K, bool shared) {
 // row LayerNorm follows as its own pass.  K = 384 (O-proj): the
 // weight-resident kernel above the rows of the carried LayerNorms (8704 /
 // 15360 / 20480 / 65536 rows 12.1 / 13.1 / 16.9 / 37.6 us against 13.0 / 15.0 /
-// 19.3 / 46.3 for the best tile).  Wider K (FFN2): whole-row tiles once tile 40
-// needs a second round of workgroups (8704 / 10240 rows: 16.3 / 17.3 us and a
-// 5.5-6 us pass against 30.4 / 31.0 on 64x384; 15360: 27.6 and 7.5 against
-// 33.3).
+// 19.3 / 46.3 for the best tile).  Wider K (FFN2): whole-row tiles from the
+// same row count, slower up to 10880 rows than tile 40 and a pass (8704 / 10240
+// rows: 16.3 / 17.3 us and a 5.5-6 us pass against 30.4 / 31.0 on 64x384), but
+// there the sums a pass would read back as fp16 stay in fp32.
 int gemm_residual_ln_tile(int M, int K, bool* fused_ln, bool shared) {
-  *fused_ln = K == wres::K ? M > 8192 : M > std::max(8192, kCus / 3 * 128);
+  *fused_ln = M > 8192;
   if (!*fused_ln) return pick_plain(M, kHidden, K, shared);
   if (K == wres::K) return kTiles;
   return M <= 16384 ? 14 : K >= 1024 ? 18 : 28;

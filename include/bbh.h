@@ -254,9 +254,9 @@ bbh_status bbh_embed_each(bbh_pool *pool, const bbh_model *m, const int32_t *ids
  * src/model/forward.cu:20-43).  Padding rows never reach a pooled embedding
  * (masked keys get zero weight, masked queries are left out of the mean), so
  * each embedding is the one bbh_embed_batches computes: bit for bit while
- * both forwards take the same LayerNorm path (forwards of up to 8192, up to
- * 10880, up to 65535 and more rows take different ones), else to within the
- * rounding of the LayerNorm row statistics.  A sentence of length 0 gets a zero embedding.
+ * both forwards take the same LayerNorm path (a forward of more than 8192
+ * rows fuses it into the GEMM epilogue), else to within the rounding of the
+ * LayerNorm row statistics.  A sentence of length 0 gets a zero embedding.
  * Sentences are split, in order, into one forward per slot of about
  * equal token counts (more if a forward would exceed a workspace's
  * max_batch*max_seq tokens or sentences); seqs need not be multiples of 16.

@@ -376,6 +376,27 @@ def test_unfused_attention_pieces_match_fused(torch_cuda):
     assert np.abs(_np(fused) - _np(merged)).max() <= TOL
 
 
+@pytest.mark.parametrize("K", [384, 1536])
+def test_residual_layernorm_rows_above_8192(torch_cuda, K):
+    # From 8193 rows on the row sums are normalised in fp32, by whichever
+    # kernel: the rows of any such call are, bit for bit, those of a call with
+    # 70000 rows (a pass over fp16 sums would differ).
+    torch = torch_cuda
+    from bbh import engine
+
+    g = torch.Generator(device="cuda").manual_seed(K)
+    r = lambda *s: torch.randn(s, device="cuda", generator=g).half()  # noqa: E731
+    A, R = r(70000, K), r(70000, 384)
+    W, b, gm, be = (r(384, K) / K ** 0.5).half(), r(384), r(384), r(384)
+    ref = torch.empty_like(R)
+    engine.launch_linear_residual_layernorm(A, W, b, R, gm, be, ref, 70000, K)
+    for M in (8193, 8705, 10881, 16384, 16385, 50000):
+        y = torch.full((M + 1, 384), 7.0, dtype=torch.float16, device="cuda")
+        engine.launch_linear_residual_layernorm(A, W, b, R, gm, be, y, M, K)
+        assert torch.equal(y[:M], ref[:M]), M
+        assert torch.all(y[M] == 7.0)
+
+
 @pytest.mark.parametrize("N,K,Ms", [
     # The one-workgroup-per-CU tiles: at most 256 workgroups of 32x64, 64x64,
     # 96x64, 128x64, 96x128 and 128x128 (K >= 1024), each at its last row count
