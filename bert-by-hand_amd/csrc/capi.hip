@@ -140,6 +140,7 @@ struct bbh_model {
     // layer 0) in the same order.
     const f16* qkv_wp = nullptr;
     const float *qkv_fsp = nullptr, *qkv_fcp = nullptr;
+    const f16* f2_ws = nullptr;  // f2_w in 32-wide K slices (bbh::gemm_residual_ln)
   } layers[BBH_NUM_LAYERS];
 };
 
@@ -208,6 +209,7 @@ float f16_bits_to_float(uint16_t b) {
 // host copy of the weights, into one device allocation: fs and fc in fp32
 // (sums in double), W' = fp16(W * gamma) (the fp32 product of two fp16
 // values is exact, so one rounding) only where gamma is not all ones.
+// Also the weights laid out for single kernels: head-major QKV, sliced FFN2.
 bbh_status fold_operands(const std::vector<uint16_t>& host, bbh_model* m) {
   const BlobLayout& L = layout();
   const size_t H = BBH_HIDDEN;
@@ -251,7 +253,16 @@ bbh_status fold_operands(const std::vector<uint16_t>& host, bbh_model* m) {
     cur = align256(cur + 3 * H * H * sizeof(f16));
     cur = align256(cur + 2 * 3 * H * sizeof(float));
   }
+  // FFN2's W per layer, in 32-wide K slices.
+  const size_t F = BBH_FFN_DIM, f2_at = cur;
+  cur += BBH_NUM_LAYERS * H * F * sizeof(f16);
   std::vector<unsigned char> buf(cur, 0);
+  for (size_t i = 0; i < (size_t)BBH_NUM_LAYERS; ++i) {
+    const uint16_t* W = host.data() + L.off[kEmbParams + i * kPerLayer + 12];
+    uint16_t* ws = reinterpret_cast<uint16_t*>(buf.data() + f2_at) + i * H * F;
+    for (size_t k = 0; k < F; k += 32)
+      for (size_t n = 0; n < H; ++n) memcpy(ws + (k / 32 * H + n) * 32, W + n * F + k, 32 * sizeof(f16));
+  }
   for (size_t f = 0; f < folds.size(); ++f) {
     const Fold& fd = folds[f];
     const uint16_t* W = host.data() + L.off[fd.w];
@@ -317,6 +328,7 @@ bbh_status fold_operands(const std::vector<uint16_t>& host, bbh_model* m) {
     l.qkv_wp = reinterpret_cast<const f16*>(base + hm_at[i]);
     l.qkv_fsp = reinterpret_cast<const float*>(base + align256(hm_at[i] + 3 * H * H * sizeof(f16)));
     l.qkv_fcp = l.qkv_fsp + 3 * H;
+    l.f2_ws = reinterpret_cast<const f16*>(base + f2_at) + i * H * F;
   }
   for (size_t f = 0; f < folds.size(); ++f) {
     auto& l = m->layers[folds[f].layer];
@@ -472,14 +484,15 @@ struct Packed {
 bbh_status linear_residual_ln(OpTimer* t, hipStream_t s, int op, const f16* A, const f16* W,
                               const f16* bias, const f16* residual, const f16* gamma,
                               const f16* beta, f16* out, int M, int K, const char* what,
-                              bool shared, bool* ln_deferred = nullptr) {
+                              bool shared, const f16* W_slices = nullptr,
+                              bool* ln_deferred = nullptr) {
   const int H = BBH_HIDDEN;
   bool fused;
-  const int tile = bbh::gemm_residual_ln_tile(M, K, &fused, shared);
+  const int tile = bbh::gemm_residual_ln_tile(M, K, &fused, shared, W_slices != nullptr);
   if (fused)
     return timed_op(t, s, {op, tile, 1, M, H, K, 0.f}, [&] {
       return check_launch(bbh::gemm_residual_ln(A, W, bias, residual, gamma, beta, out, M, K,
-                                                BBH_LAYER_NORM_EPS, s, shared),
+                                                BBH_LAYER_NORM_EPS, s, shared, W_slices),
                           what);
     });
   BBH_TRY(timed_op(t, s, {op, tile, 0, M, H, K, 0.f}, [&] {
@@ -559,7 +572,7 @@ bbh_status run_ffn_rows(bbh_workspace* ws, const bbh_model::Layer& L, const f16*
                         "ffn1 gemm");
   }));
   return linear_residual_ln(t, s, BBH_OP_FFN2_LN, ws->inter, L.f2_w, L.f2_b, hidden, L.ln2_g,
-                            L.ln2_b, out, M, F, "ffn2 gemm+ln", ws->shared, ln_deferred);
+                            L.ln2_b, out, M, F, "ffn2 gemm+ln", ws->shared, L.f2_ws, ln_deferred);
 }
 
 bbh_status run_ffn_block(bbh_workspace* ws, const bbh_model::Layer& L, const f16* hidden,

@@ -51,10 +51,14 @@ struct Cfg {
   // PD_ > 0: register prefetch depth (mainloop_reg).  PD_ = -(16 NP + KPB):
   // one ring of whole slices (mainloop_deep), KPB of them per barrier, copied
   // by NP wavefronts of their own beside the WM x WN that compute (NP = 0: by
-  // those); 256 more: slices 32 wide instead of 64.
+  // those); 256 more: slices 32 wide instead of 64, and W laid out slice by
+  // slice (W_SLICES: element (n, k) at (k / 32 * N + n) * 32 + k % 32, N = BN).
+  // Row-major, a 32-wide slice would fetch every 128-byte line of W twice, half
+  // a line each: the copies, not the MFMAs, set the pace of such a tile.
   static constexpr int PD = PD_ > 0 ? PD_ : 0;
   static constexpr int KPB = PD_ < 0 ? -PD_ % 16 : 1, NP = PD_ < 0 ? -PD_ / 16 % 16 : 0;
   static constexpr int BK = -PD_ >= 256 ? 32 : 64, RPC = 512 / BK;  // rows of a 1 KB copy
+  static constexpr bool W_SLICES = BK == 32;
   using L = Slice<BK>;
   static constexpr int NW = WM * WN, THREADS = 64 * (NW + NP);
   static constexpr int NC = NP > 0 ? NP : NW;            // wavefronts that issue the copies
@@ -90,7 +94,8 @@ struct Cfg {
 
 // Copying one 64-wide K slice of ROWS K-contiguous rows into LDS: each
 // wavefront instruction fills 1 KB = 8 rows (16 of a 32-wide slice); lane i
-// lands at row i / 8, slot i % 8 of them, so it fetches the logical chunk that belongs in that slot.
+// lands at row i / 8, slot i % 8 of them (i / 4, i % 4), so it fetches the
+// logical chunk that belongs in that slot.
 // Rows at or past `valid` are read clamped to row valid-1.  row_offsets gives
 // off[j] = byte offset of this lane's chunk of copy j from the slice base,
 // computed once per tile; issue_rows_at then copies a slice through a buffer
@@ -323,7 +328,7 @@ __device__ __forceinline__ void mainloop_deep(const f16* __restrict__ A,
   const __amdgpu_buffer_rsrc_t rA = buffer_of(A + (size_t)m0 * K, (uint32_t)(M - m0) * K * 2u);
   const __amdgpu_buffer_rsrc_t rW = buffer_of(W + (size_t)n0 * K, (uint32_t)C::BN * K * 2u);
   auto issue = [&](int s, int slot) {
-    issue_rows_at(rW, s * C::BK * 2, offW, ringW + slot * C::W_STAGE, cw);
+    issue_rows_at(rW, s * (C::W_SLICES ? C::W_STAGE : C::BK) * 2, offW, ringW + slot * C::W_STAGE, cw);
     issue_rows_at(rA, s * C::BK * 2, offA, ringA + slot * C::A_STAGE, cw);
   };
   int slot = 0;  // of slice kt
@@ -340,7 +345,7 @@ __device__ __forceinline__ void mainloop_deep(const f16* __restrict__ A,
   };
   if (copies) {
     row_offsets<C::BM, C::NC, C::BK>(K, M - m0, offA, cw);
-    row_offsets<C::BN, C::NC, C::BK>(K, C::BN, offW, cw);
+    row_offsets<C::BN, C::NC, C::BK>(C::W_SLICES ? C::BK : K, C::BN, offW, cw);
 #pragma unroll
     for (int d = 0; d < R - P; ++d)
       if (d < KT) issue(d, d);
@@ -1647,7 +1652,7 @@ hipError_t launch(const f16* A, const f16* W, const f16* bias, const f16* residu
 }
 
 // Tile configurations (BM, BN, wavefronts M x N, A-ring depth), by id; the K
-// slice is 64 wide and the W ring 2 deep but in tiles 35-41.  The product build holds
+// slice is 64 wide and the W ring 2 deep but in tiles 35-42.  The product build holds
 // the configurations pick_plain and gemm_residual_ln_tile choose; the others
 // of the sweep that chose them are compiled only with -DBBH_TUNING.
 //   id  tile      wave tile  SA   LDS
@@ -1671,6 +1676,8 @@ hipError_t launch(const f16* A, const f16* W, const f16* bias, const f16* residu
 //   39  96x128    32x64 (6w) 4    112 KB   NP 4
 //   40  128x128   64x64      4    128 KB   NP 4
 //   41  64x128    32x32 (8w) 3     72 KB   NP 0
+//   42  64x384    64x96      5    140 KB   NP 4, 32-wide slices, sliced W
+//       (owns whole rows; kSlicedTile, launched by gemm_residual_ln only)
 // Kernel symbols read gemm_kernel<Cfg<BM,BN,WM,WN,SA,PD,SW>, epilogue>.
 // The table itself: X(id, BM, BN, WM, WN, SA, PD, SW).
 #define BBH_TILES(X) \
@@ -1733,9 +1740,14 @@ struct TileOf;
     using type = Cfg<BM, BN, WM, WN, SA, PD, SW>;     \
   };
 BBH_TILES(BBH_TILE_TYPE)
-#undef BBH_TILE_TYPE
 template <int ID>
 using TileCfg = typename TileOf<ID>::type;
+
+// FFN2 + LayerNorm from W laid out in 32-wide slices (tile 42).
+#define BBH_SLICED(X) X(42, 64, 384, 1, 4, 5, -321, 5)
+constexpr int kSlicedTile = 42;
+BBH_SLICED(BBH_TILE_TYPE)
+#undef BBH_TILE_TYPE
 
 template <int EPI>
 hipError_t launch_id(int id, const f16* A, const f16* W, const f16* bias, const f16* residual,
@@ -1771,6 +1783,7 @@ const char* tile_name(int id) {
     return "Cfg<" #BM "," #BN "," #WM "," #WN "," #SA "," #PD "," #SW ">";
   switch (id) {
     BBH_TILES(BBH_NAME)
+    BBH_SLICED(BBH_NAME)
     BBH_TUNING_TILES(BBH_NAME)
   }
 #undef BBH_NAME
@@ -1884,11 +1897,16 @@ int gemm_tile(int M, int N, int K, bool shared) {
 // 19.3 / 46.3 for the best tile).  Wider K (FFN2): whole-row tiles from the
 // same row count, slower up to 10880 rows than tile 40 and a pass (8704 / 10240
 // rows: 16.3 / 17.3 us and a 5.5-6 us pass against 30.4 / 31.0 on 64x384), but
-// there the sums a pass would read back as fp16 stay in fp32.
-int gemm_residual_ln_tile(int M, int K, bool* fused_ln, bool shared) {
+// there the sums a pass would read back as fp16 stay in fp32.  Where the
+// caller holds W in slices too (a model does), tile 42 as long as one
+// workgroup per CU covers the rows: 9216 / 12288 / 15360 rows 30.1 / 31.5 /
+// 32.8 -> 23.7 / 25.4 / 27.6 us; its two rounds at 20480 rows take 47.7 against
+// 38.1 on tile 18.
+int gemm_residual_ln_tile(int M, int K, bool* fused_ln, bool shared, bool sliced) {
   *fused_ln = M > 8192;
   if (!*fused_ln) return pick_plain(M, kHidden, K, shared);
   if (K == wres::K) return kTiles;
+  if (sliced && M <= kCus * TileCfg<kSlicedTile>::BM) return kSlicedTile;
   return M <= 16384 ? 14 : K >= 1024 ? 18 : 28;
 }
 
@@ -1918,9 +1936,12 @@ hipError_t gemm(const f16* A, const f16* W, const f16* bias, f16* C, int M, int 
 
 hipError_t gemm_residual_ln(const f16* A, const f16* W, const f16* bias, const f16* residual,
                             const f16* gamma, const f16* beta, f16* y, int M, int K, float eps,
-                            hipStream_t s, bool shared) {
+                            hipStream_t s, bool shared, const f16* W_slices) {
   bool fused;
-  const int id = gemm_residual_ln_tile(M, K, &fused, shared);
+  const int id = gemm_residual_ln_tile(M, K, &fused, shared, W_slices != nullptr);
+  if (id == kSlicedTile)
+    return launch<TileCfg<kSlicedTile>, kLayerNorm>(A, W_slices, bias, residual, gamma, beta, y, M,
+                                                    kHidden, K, eps, s);
   if (id == kTiles)
     return launch_wres<kLayerNorm>(A, W, bias, y, M, kHidden, s, residual, gamma, beta, eps);
   if (fused)

@@ -73,15 +73,17 @@ hipError_t qkv_attention(const f16* X, const f16* Wp, const float* fs, const flo
 // plain tiled kernel), whether the LayerNorm is inside the GEMM kernel, and
 // the configuration's name as it appears in the kernel symbol.
 int gemm_tile(int M, int N, int K, bool shared = false);
-int gemm_residual_ln_tile(int M, int K, bool* fused_ln, bool shared = false);
+int gemm_residual_ln_tile(int M, int K, bool* fused_ln, bool shared = false, bool sliced = false);
 const char* gemm_tile_name(int tile);
 
 // y(M,384) = LN(A(M,K) . W(384,K)^T + bias + residual) * gamma + beta.
-// y may alias residual.  K % 64 == 0.
+// y may alias residual.  K % 64 == 0.  W_slices: W again, where the caller
+// holds it in 32-wide K slices (element (n, k) at (k / 32 * 384 + n) * 32 + k % 32),
+// else null; same result.
 hipError_t gemm_residual_ln(const f16* A, const f16* W, const f16* bias,
                             const f16* residual, const f16* gamma, const f16* beta,
                             f16* y, int M, int K, float eps, hipStream_t s,
-                            bool shared = false);
+                            bool shared = false, const f16* W_slices = nullptr);
 
 // The first half of gemm_residual_ln where gemm_residual_ln_tile says the
 // LayerNorm is not fused: y = A . W^T + bias + residual (fp16), which a

@@ -578,6 +578,34 @@ def test_pool_normalize(torch_cuda, B, S):
         assert np.all(got[2] == 0.0)
 
 
+@pytest.mark.parametrize("B,S", [(256, 32), (171, 48), (95, 96), (113, 144), (256, 64), (205, 80)])
+def test_ffn_block_from_sliced_weights(torch_cuda, ws, model, weights32, B, S):
+    # 8192 to 16400 rows: above 8192 and up to 16384 ffn_block reads FFN2's weights
+    # from the model's sliced copy, the standalone launchers read them
+    # row-major.  Same bits, and no row past the last one written.
+    from bbh import engine
+
+    torch = torch_cuda
+    M = B * S
+    g = torch.Generator(device="cuda").manual_seed(M)
+    hid = torch.randn((M, 384), device="cuda", generator=g).half()
+    for i in (0, 5):
+        p = "encoder.layer.%d." % i
+        w = {k[len(p):]: to_dev(torch, v.astype(np.float16)) for k, v in weights32.items()
+             if k.startswith(p)}
+        inter = torch.empty((M, 1536), dtype=torch.float16, device="cuda")
+        engine.launch_matmul(hid, w["intermediate.dense.weight"], inter, M, 1536, 384,
+                             bias=w["intermediate.dense.bias"], gelu=True)
+        want = torch.empty_like(hid)
+        engine.launch_linear_residual_layernorm(
+            inter, w["output.dense.weight"], w["output.dense.bias"], hid,
+            w["output.LayerNorm.weight"], w["output.LayerNorm.bias"], want, M, 1536)
+        out = torch.full((M + 1, 384), 7.0, dtype=torch.float16, device="cuda")
+        engine.ffn_block(ws, model, i, hid, out, B, S)
+        assert torch.equal(out[:M], want)
+        assert torch.all(out[M] == 7.0)
+
+
 @pytest.mark.parametrize("B,S", [(4097, 16), (192, 512), (256, 512)])
 def test_ffn_one_kernel_equals_two_kernels(torch_cuda, ws, model, weights32, weights16, B, S):
     # From 65536 rows bbh_ffn_block runs the FFN as one kernel (intermediate
