@@ -1803,9 +1803,8 @@ const char* tile_name(int id) {
 // 64x64 copy-ring tile (0) up to 2048 rows (2048 rows: 6.4 us against 6.9 on
 // tile 30), FFN1 to 4096 rows (one-slot pass 8.22-8.24 -> 8.11 ms against the
 // register-staged 64x64 at 2049-3072 rows): more workgroups than CUs keep
-// every CU busy.  At 6145-8192 rows alone FFN1 takes tile 31 and O-proj tile
-// 0 (configs[2] forward 387.5 -> 383.5 us on one box, every repeat; level on
-// a slower one).
+// every CU busy.  At 4097-8192 rows alone FFN1 takes 256x192 (19), which
+// covers 8192 rows with one workgroup per CU, and O-proj past pick_deep tile 0.
 // Beside other forwards (shared true: a pool of several slots) every tile was
 // tried for each (shape, M) with the others fixed in the per-batch pass, then
 // the winners confirmed in interleaved repeats: FFN1 takes the 128x128
