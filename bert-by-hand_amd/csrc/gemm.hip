@@ -1890,10 +1890,12 @@ int gemm_tile(int M, int N, int K, bool shared) {
 // Large M: one kernel that owns whole rows.  Smaller M: a tile that owns whole
 // rows leaves most CUs idle and streams all of W per workgroup, so the GEMM
 // runs on 2-D tiles with a bias + residual epilogue (in place over y) and the
-// row LayerNorm follows as its own pass.  K = 384 (O-proj): the
-// weight-resident kernel above the rows of the carried LayerNorms (8704 /
-// 15360 / 20480 / 65536 rows 12.1 / 13.1 / 16.9 / 37.6 us against 13.0 / 15.0 /
-// 19.3 / 46.3 for the best tile).  Wider K (FFN2): whole-row tiles from the
+// row LayerNorm follows as its own pass.  K = 384 (O-proj): tiles 14 and 28,
+// from 65536 rows the weight-resident kernel (37.6 us against 46.3 there).  It
+// would be faster from 8193 rows on (8704 / 15360 / 20480 rows 12.1 / 13.1 /
+// 16.9 us against 13.0 / 15.0 / 19.3), but it adds a row's statistics up from 12
+// groups of 32 columns instead of 4 of 96: as exact, but other last bits than
+// these row counts have always given, 3e-4 of a packed corpus' embeddings.  Wider K (FFN2): whole-row tiles from the
 // same row count, slower up to 10880 rows than tile 40 and a pass (8704 / 10240
 // rows: 16.3 / 17.3 us and a 5.5-6 us pass against 30.4 / 31.0 on 64x384), but
 // there the sums a pass would read back as fp16 stay in fp32.  Where the
@@ -1904,7 +1906,7 @@ int gemm_tile(int M, int N, int K, bool shared) {
 int gemm_residual_ln_tile(int M, int K, bool* fused_ln, bool shared, bool sliced) {
   *fused_ln = M > 8192;
   if (!*fused_ln) return pick_plain(M, kHidden, K, shared);
-  if (K == wres::K) return kTiles;
+  if (K == wres::K && M >= 65536) return kTiles;
   if (sliced && M <= kCus * TileCfg<kSlicedTile>::BM) return kSlicedTile;
   return M <= 16384 ? 14 : K >= 1024 ? 18 : 28;
 }

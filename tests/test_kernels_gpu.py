@@ -380,7 +380,9 @@ def test_unfused_attention_pieces_match_fused(torch_cuda):
 def test_residual_layernorm_rows_above_8192(torch_cuda, K):
     # From 8193 rows on the row sums are normalised in fp32, by whichever
     # kernel: the rows of any such call are, bit for bit, those of a call with
-    # 70000 rows (a pass over fp16 sums would differ).
+    # 65535 rows (a pass over fp16 sums would differ); K = 1536 those of one
+    # with 70000 rows too.  (K = 384 runs on the weight-resident kernel from
+    # 65536 rows on, which groups the columns of a row's statistics otherwise.)
     torch = torch_cuda
     from bbh import engine
 
@@ -388,8 +390,8 @@ def test_residual_layernorm_rows_above_8192(torch_cuda, K):
     r = lambda *s: torch.randn(s, device="cuda", generator=g).half()  # noqa: E731
     A, R = r(70000, K), r(70000, 384)
     W, b, gm, be = (r(384, K) / K ** 0.5).half(), r(384), r(384), r(384)
-    ref = torch.empty_like(R)
-    engine.launch_linear_residual_layernorm(A, W, b, R, gm, be, ref, 70000, K)
+    ref, rows = torch.empty_like(R), 65535 if K == 384 else 70000
+    engine.launch_linear_residual_layernorm(A, W, b, R, gm, be, ref, rows, K)
     for M in (8193, 8705, 10881, 16384, 16385, 50000):
         y = torch.full((M + 1, 384), 7.0, dtype=torch.float16, device="cuda")
         engine.launch_linear_residual_layernorm(A, W, b, R, gm, be, y, M, K)

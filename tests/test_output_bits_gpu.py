@@ -1,0 +1,72 @@
+"""Outputs that stay the same bits from version to version (GPU).
+
+The order of the sums in a row's LayerNorm shows in the last bit of an fp16
+output, and through six layers in the embedding.  A kernel or a rule on sizes
+that changes it changes what users have stored, so the outputs below are pinned
+by checksum at sizes on both sides of every such rule.  Inputs come from seeded
+numpy.
+"""
+import zlib
+
+import numpy as np
+import pytest
+from conftest import to_dev
+
+pytestmark = pytest.mark.gpu
+
+# (rows, K) of Linear + residual + LayerNorm
+RESIDUAL_LN = {(8192, 384): 4054097961, (8193, 384): 1293971833, (16384, 384): 1677011260,
+    (16385, 384): 1138506625, (30001, 384): 3859647307, (65535, 384): 476011240,
+    (65536, 384): 652312738, (8193, 1536): 2831042692, (16385, 1536): 3336549077}
+# (sentences, seq) of packed forwards: below and above 8192 rows
+PACKED = {(150, 64): 2387981691, (300, 64): 3287569568, (700, 64): 3720832445}
+
+
+def _crc(t):
+    return zlib.crc32(t.cpu().numpy().tobytes())
+
+
+def residual_ln_crc(torch, M, K):
+    from bbh import engine
+
+    rng = np.random.default_rng(M + K)
+    h = lambda *s: rng.standard_normal(s, dtype=np.float32)  # noqa: E731
+    A, W, R = h(M, K), h(384, K) / np.float32(K ** 0.5), h(M, 384)
+    b, g, be = h(384), 1 + h(384) / 4, h(384) / 8
+    A, W, R, b, g, be = (to_dev(torch, x.astype(np.float16)) for x in (A, W, R, b, g, be))
+    y = torch.empty_like(R)
+    engine.launch_linear_residual_layernorm(A, W, b, R, g, be, y, M, K)
+    return _crc(y)
+
+
+def packed_crc(torch, B, S):
+    from bbh import engine, synth
+
+    w = synth.make_weights(0)
+    rng = np.random.default_rng(B + S)
+    for k in sorted(w):  # peaked attention, LayerNorms that are not the identity
+        if k.endswith("LayerNorm.weight"):
+            w[k] = rng.uniform(0.6, 1.4, w[k].shape).astype(np.float32)
+        elif ".query.weight" in k or ".key.weight" in k:
+            w[k] = w[k] * 4
+    model = engine.Model.from_weights(w)
+    n = rng.integers(S // 4, S + 1, size=B)
+    mask = (np.arange(S)[None] < n[:, None]).astype(np.int32)
+    ids = (rng.integers(1000, 30522, size=(B, S)) * mask).astype(np.int32)
+    pool = engine.Pool(1, B, S)
+    out = engine.embed_packed(pool, model, engine.PackedBatches([(ids, np.zeros_like(ids), mask)]))
+    torch.cuda.synchronize()
+    crc = _crc(out)
+    pool.close()
+    model.close()
+    return crc
+
+
+@pytest.mark.parametrize("M,K", RESIDUAL_LN)
+def test_residual_layernorm_bits(torch_cuda, M, K):
+    assert residual_ln_crc(torch_cuda, M, K) == RESIDUAL_LN[M, K]
+
+
+@pytest.mark.parametrize("B,S", PACKED)
+def test_packed_bits(torch_cuda, B, S):
+    assert packed_crc(torch_cuda, B, S) == PACKED[B, S]
