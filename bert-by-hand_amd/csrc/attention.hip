@@ -36,7 +36,7 @@
 // Short sequences are bound by the global round trip: all of a workgroup's
 // loads (Q, K, V, mask) are issued before its single barrier, and the output
 // goes out through LDS as 16-byte stores of 64 contiguous bytes per row.
-// Long sequences are bound by exp + MFMA issue; at 16 tiles a wavefront takes
+// Long sequences are bound by exp + MFMA issue; at 8 and 16 tiles a wavefront takes
 // two query tiles at once, sharing each K and V^T operand read between them.
 
 #include <algorithm>
@@ -207,6 +207,7 @@ __global__ __launch_bounds__(64 * NW, T == 2 || NW > 8 ? 4 : 6) void attention_k
         }
       }
       float mx[T];
+      bool up = false;
 #pragma unroll
       for (int t = 0; t < T; ++t) {
         // IEEE maximum (v_maximum3_f32): scores hold no NaN, and unlike fmaxf
@@ -221,21 +222,21 @@ __global__ __launch_bounds__(64 * NW, T == 2 || NW > 8 ? 4 : 6) void attention_k
                                                          false, false);
         mx[t] = __builtin_elementwise_maximum(__uint_as_float(sw[0]),
                                               __uint_as_float(sw[1]));  // finite: a key is unmasked
+        up = up || mx[t] > m[t] + lag;
       }
       if (!started) {
 #pragma unroll
         for (int t = 0; t < T; ++t) m[t] = mx[t];
         started = true;
-      } else {  // each tile for itself, so its bits do not depend on T
+      } else if (__ballot(up)) {  // the tiles of a group together
 #pragma unroll
-        for (int t = 0; t < T; ++t)
-          if (__ballot(mx[t] > m[t] + lag)) {
-            const float mn = fmaxf(m[t], mx[t]);
-            const float corr = __builtin_amdgcn_exp2f((m[t] - mn) * c);
-            l[t] *= corr;
-            o[t] *= corr;
-            m[t] = mn;
-          }
+        for (int t = 0; t < T; ++t) {
+          const float mn = fmaxf(m[t], mx[t]);
+          const float corr = __builtin_amdgcn_exp2f((m[t] - mn) * c);
+          l[t] *= corr;
+          o[t] *= corr;
+          m[t] = mn;
+        }
       }
       const f16* vrow = Vt + r32 * VLD + kc * 32 + 8 * kh;
       const f16x8 va = *reinterpret_cast<const f16x8*>(vrow);
@@ -333,18 +334,23 @@ hipError_t launch_attention(const f16* qkv, const int32_t* mask, f16* merged, in
 }
 
 // Workgroup shape by query-tile count (tiles = ceil(seq / 32); for packed
-// sentences of the longest one).  2-4 tiles: 4 wavefronts of one tile each,
-// output staged through the K/V area.  5-8: 8 wavefronts, 9-16: 12, one tile at
-// a time and stored straight from the accumulators: more wavefronts than
-// tiles still help to stage K and V, and more of them hide the exp and MFMA
-// latencies than 4 or 8, or two tiles a wavefront (266 x 96 21.2 -> 17.6 us, 600
-// x 64 23.6 -> 22.1, 64 x 144 / 192 / 256 11.2 / 13.7 / 19.5 -> 9.0 / 12.5 /
-// 18.6, 21 x 304 12.5 -> 11.3, 80 x 288 / 480 28.0 / 54.9 -> 27.1 / 52.3, 128 x
-// 512 85.6 -> 81.2).  Where a CU's share of workgroups fills it anyway: 9-11
-// tiles on 8 wavefronts (three workgroups a CU against two: 160 x 288 47.2 ->
-// 44.9), 16 on 8 x 2, each operand read serving two tiles, output staged (256
-// x 512 174 -> 172).  Packed sentences of up to 3 tiles: 2 wavefronts, for most
-// sentences are much shorter than the longest.
+// sentences of the longest one).
+//  - 2-4 tiles: 4 wavefronts of one tile each, output staged through the K/V
+//    area (266 x 96 21.2 -> 17.6 us, 600 x 64 23.6 -> 22.1 against one wavefront
+//    a tile).  Packed sentences of up to 3 tiles: 2 wavefronts, for most
+//    sentences are much shorter than the longest.
+//  - 8 and 16 tiles: 4 and 8 wavefronts of two tiles, output staged.  The two
+//    tiles of a wavefront are rescaled together, which shows in the last bits,
+//    so these counts take this shape in every batch (one tile a wavefront: 512 x
+//    256 129 us against 122 here, 128 x 512 96 against 94, but 64 x 256 20.7
+//    against 21.2).
+//  - Else 5-7 tiles: 8 wavefronts, 9-15: 12, one tile at a time and stored
+//    straight from the accumulators: more wavefronts than tiles still help to
+//    stage K and V, and more of them hide the exp and MFMA latencies than 4 or
+//    8 (64 x 144 / 192 11.2 / 13.7 -> 9.0 / 12.5 us, 21 x 304 12.5 -> 11.3, 80 x
+//    288 / 480 28.0 / 54.9 -> 27.1 / 52.3).  Where a CU's share of workgroups
+//    fills it anyway, 9-11 tiles on 8 wavefronts (three workgroups a CU against
+//    two: 160 x 288 47.2 -> 44.9).
 template <bool VL>
 hipError_t attention_any(const f16* qkv, const int32_t* mask, f16* merged, int batch, int heads,
                          int seq, float scale, hipStream_t s, const PackedSentence* sents) {
@@ -353,7 +359,8 @@ hipError_t attention_any(const f16* qkv, const int32_t* mask, f16* merged, int b
 #define BBH_ATT(NW, T, F) \
   launch_attention<NW, T, F, VL>(qkv, mask, merged, batch, heads, seq, c, s, sents)
   const int wgs = batch * heads;
-  if (tiles >= 16 && wgs > 2048) return BBH_ATT(8, 2, 3);
+  if (tiles >= 16) return BBH_ATT(8, 2, 3);
+  if (tiles == 8) return BBH_ATT(4, 2, 3);
   if (tiles > (wgs > 1280 ? 11 : 8)) return BBH_ATT(12, 1, 0);
   if (tiles > 4) return BBH_ATT(8, 1, 0);
   if (tiles >= (VL ? 4 : 2)) return BBH_ATT(4, 1, 3);

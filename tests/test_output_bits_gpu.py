@@ -1,10 +1,11 @@
 """Outputs that stay the same bits from version to version (GPU).
 
-The order of the sums in a row's LayerNorm shows in the last bit of an fp16
-output, and through six layers in the embedding.  A kernel or a rule on sizes
-that changes it changes what users have stored, so the outputs below are pinned
-by checksum at sizes on both sides of every such rule.  Inputs come from seeded
-numpy.
+The order of the sums in a row's LayerNorm and the softmax's rescale decisions
+show in the last bit of an fp16 output, and through six layers in the embedding.
+A kernel, a workgroup shape or a rule on sizes that changes them changes what
+users have stored, so the outputs below are pinned by checksum at sizes on both
+sides of every such rule.  Inputs come from seeded numpy; scores rise along the
+keys, so that the running maximum moves often.
 """
 import zlib
 
@@ -14,16 +15,39 @@ from conftest import to_dev
 
 pytestmark = pytest.mark.gpu
 
+# (sentences, seq): 1 to 16 query tiles, the tile counts at which two tiles share
+# a wavefront (8 and 16) in small and large batches, and the batches past which
+# 9-11 tiles take other workgroups.
+ATTENTION = {(3, 16): 508316586, (3, 112): 3209609789, (2, 240): 3976281866,
+    (40, 256): 134725881, (5, 288): 2063144199, (110, 288): 2336928259, (108, 352): 205674545,
+    (2, 400): 3171030908, (2, 496): 3040453196, (3, 512): 3132702209, (172, 496): 481132825,
+    (172, 512): 3705176780}
 # (rows, K) of Linear + residual + LayerNorm
 RESIDUAL_LN = {(8192, 384): 4054097961, (8193, 384): 1293971833, (16384, 384): 1677011260,
     (16385, 384): 1138506625, (30001, 384): 3859647307, (65535, 384): 476011240,
     (65536, 384): 652312738, (8193, 1536): 2831042692, (16385, 1536): 3336549077}
-# (sentences, seq) of packed forwards: below and above 8192 rows
-PACKED = {(150, 64): 2387981691, (300, 64): 3287569568, (700, 64): 3720832445}
+# (sentences, seq) of packed forwards: below and above 8192 rows, long sentences
+PACKED = {(150, 64): 2387981691, (300, 64): 3287569568, (700, 64): 3720832445,
+    (60, 512): 631409041}
 
 
 def _crc(t):
     return zlib.crc32(t.cpu().numpy().tobytes())
+
+
+def attention_crc(torch, B, S):
+    from bbh import engine
+
+    rng = np.random.default_rng(100 * B + S)
+    qkv = (2.0 * rng.standard_normal((B, S, 1152))).astype(np.float32)
+    qkv[:, :, 384:768] += np.arange(S, dtype=np.float32)[None, :, None] * 0.02
+    n = rng.integers(1, S + 1, size=B)
+    n[0] = S
+    mask = (np.arange(S)[None] < n[:, None]).astype(np.int32)
+    out = torch.empty((B * S, 384), dtype=torch.float16, device="cuda")
+    engine.launch_attention(to_dev(torch, qkv.astype(np.float16).reshape(B * S, 1152)),
+                            to_dev(torch, mask), out, B, S)
+    return _crc(out)
 
 
 def residual_ln_crc(torch, M, K):
@@ -60,6 +84,11 @@ def packed_crc(torch, B, S):
     pool.close()
     model.close()
     return crc
+
+
+@pytest.mark.parametrize("B,S", ATTENTION)
+def test_attention_bits(torch_cuda, B, S):
+    assert attention_crc(torch_cuda, B, S) == ATTENTION[B, S]
 
 
 @pytest.mark.parametrize("M,K", RESIDUAL_LN)
