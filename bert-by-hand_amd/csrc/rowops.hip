@@ -319,12 +319,14 @@ __global__ __launch_bounds__(256) void mean_pool_kernel(const f16* __restrict__ 
   out[idx] = (f16)(acc / (float)(cnt > 0 ? cnt : 1));
 }
 
-// The same for dim % 8 == 0 up to kPoolThreads columns of eight: one
-// workgroup per sentence, eight columns a thread, the positions dealt to as
-// many row groups as the threads allow and the groups' sums added through
-// LDS.  Masked rows are not read.  Bound by the row loads' latency, four of
-// which a thread keeps in flight: 128 x 112 rows of 384 took 50.6 us with one
-// thread a column walking the mask, against 6.1 us here.
+// The same for dim % 8 == 0 up to kPoolThreads columns of eight and batches
+// below 2^22 (a launch holds less than 2^32 threads; a larger one is not
+// refused, its workgroup count wraps): one workgroup per sentence, eight
+// columns a thread, the positions dealt to as many row groups as the threads
+// allow and the groups' sums added through LDS.  Masked rows are not read.
+// Bound by the row loads' latency, four of which a thread keeps in flight: 128 x
+// 112 rows of 384 took 50.6 us with one thread a column walking the mask,
+// against 6.1 us here.
 constexpr int kPoolThreads = 1024;
 __global__ __launch_bounds__(kPoolThreads) void mean_pool8_kernel(
     const f16* __restrict__ hidden, const int32_t* __restrict__ mask, f16* __restrict__ out,
@@ -468,7 +470,7 @@ hipError_t embedding_ln(const int32_t* ids, const int32_t* types, const f16* wor
 
 hipError_t mean_pool(const f16* hidden, const int32_t* mask, f16* out, int batch, int seq,
                      int dim, hipStream_t s) {
-  if (dim % 8 == 0 && dim / 8 <= kPoolThreads) {
+  if (dim % 8 == 0 && dim / 8 <= kPoolThreads && batch < (1ll << 32) / kPoolThreads) {
     const int groups = std::min(kPoolThreads / (dim / 8), seq);
     const size_t lds = (size_t)groups * (dim + 1) * sizeof(float);  // at most 36 KB
     hipLaunchKernelGGL(mean_pool8_kernel, dim3(batch), dim3(kPoolThreads), lds, s, hidden, mask,

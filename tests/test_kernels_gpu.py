@@ -514,6 +514,20 @@ def test_row_operators_edges(torch_cuda, B, S, D, off):
     assert np.all(np.abs(got - want) <= (2 ** -10 + D * 2 ** -23) * np.abs(want) + 2 ** -24)
 
 
+def test_mean_pool_of_many_short_rows(torch_cuda):
+    # More sentences than a launch of one 1024-thread workgroup each can hold
+    # (2^32 threads): every row is written, the last ones too.
+    torch = torch_cuda
+    from bbh import engine
+
+    B, D = (1 << 22) + 8, 8
+    h = (torch.arange(B, device="cuda") % 2048).half()[:, None] + torch.arange(D, device="cuda").half()
+    mask = torch.ones((B, 1), dtype=torch.int32, device="cuda")
+    out = torch.full((B, D), -1.0, dtype=torch.float16, device="cuda")
+    engine.launch_mean_pool(h, mask, out, 1, D, B)
+    assert torch.equal(out, h)  # the mean of one row
+
+
 def test_softmax_reference_kat(torch_cuda, kats):
     torch = torch_cuda
     from bbh import engine
