@@ -363,10 +363,11 @@ hipError_t attention_any(const f16* qkv, const int32_t* mask, f16* merged, int b
   if (tiles == 8) return BBH_ATT(4, 2, 3);
   if (tiles > (wgs > 1280 ? 11 : 8)) return BBH_ATT(12, 1, 0);
   if (tiles > 4) return BBH_ATT(8, 1, 0);
-  if (tiles >= (VL ? 4 : 2)) return BBH_ATT(4, 1, 3);
-  if constexpr (VL) {
-    if (tiles >= 2) return BBH_ATT(2, 1, 3);
-  }
+  // A launch holds less than 2^32 threads (a larger one is not refused, its
+  // workgroup count wraps): 2^24 workgroups and more on 2 wavefronts, too.
+  const bool fits4 = (long)xcd_grid(batch, heads) * 256 < 1l << 32;
+  if (tiles >= (VL ? 4 : 2) && fits4) return BBH_ATT(4, 1, 3);
+  if (tiles >= 2) return BBH_ATT(2, 1, 3);
   return BBH_ATT(1, 1, 3);
 #undef BBH_ATT
 }
