@@ -1559,13 +1559,22 @@ __global__ __launch_bounds__(wres::THREADS) void gemm_wres_kernel(
   }
 }
 
-// The weight-resident kernel serves K = 384 and N a multiple of 384 above the
-// rows of the carried LayerNorms, where its two passes over W per CU (the
-// prologue) are paid back.  Back to back launches against the tiles: FFN1 +
-// GELU at 8704 / 12288 / 15360 rows 23.7 / 29.2 / 34.4 -> 20.6 / 24.4 / 29.7
-// us; QKV at 10240 / 12288 / 15360 / 20480 rows 16.8 / 19.8 / 23.7 / 28.8 ->
-// 16.1 / 17.7 / 20.6 / 24.8 us.
-bool wres_ok(int M, int N, int K) { return K == wres::K && N % wres::COLS == 0 && M > 8192; }
+// The weight-resident kernel serves K = 384 and N a multiple of 384 from the rows
+// where its two passes over W per CU (the prologue) are paid back.  Back to back
+// launches against the tiles, us:
+//   N = 1536: 8193 / 10240 / 12288 / 15360 rows 16.5 / 18.4 / 21.8 / 26.1 -> 15.9 /
+//     17.7 / 19.8 / 23.5
+//   N = 1152: 8193 / 10880 / 11008 / 16384 / 20480 rows 13.8 / 15.1 / 17.3 / 22.0 /
+//     26.5 -> 14.3 / 16.5 / 16.5 / 20.9 / 23.5
+//   N = 768: 10240 / 10880 / 11008 / 16384 / 20480 rows 11.0 / 11.2 / 13.3 / 15.1 /
+//     18.8 -> 12.2 / 12.4 / 12.4 / 15.4 / 17.9
+//   N = 384: 8193 / 10880 / 16384 / 20480 / 22528 rows 7.8 / 7.8 / 10.3 / 10.9 / 13.7
+//     -> 9.5 / 9.7 / 10.2 / 12.5 / 12.9
+// 10880 rows are the last that 128x128 tiles cover in one round of two workgroups
+// a CU at N = 768, 21760 at N = 384.
+bool wres_ok(int M, int N, int K) {
+  return K == wres::K && N % wres::COLS == 0 && M > (N >= 1536 ? 8192 : N >= 768 ? 10880 : 21760);
+}
 
 template <int EPI>
 hipError_t launch_wres(const f16* A, const f16* W, const f16* bias, f16* out, int M, int N,
