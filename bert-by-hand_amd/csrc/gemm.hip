@@ -1809,11 +1809,17 @@ const char* tile_name(int id) {
 // CUs.
 // Alone (shared false: bbh_embed, a one-slot pool), pick_deep's tiles first;
 // past them, from sweeps with one GEMM's tile changed at a time: QKV runs the
-// 64x64 copy-ring tile (0) up to 2048 rows (2048 rows: 6.4 us against 6.9 on
-// tile 30), FFN1 to 4096 rows (one-slot pass 8.22-8.24 -> 8.11 ms against the
-// register-staged 64x64 at 2049-3072 rows): more workgroups than CUs keep
-// every CU busy.  At 4097-8192 rows alone FFN1 takes 256x192 (19), which
+// 64x64 copy-ring tile (0) up to 2048 rows (inside bert_embed 4 x 512 304 us
+// against 307 on tile 30, and below, on pick_deep's tiles, 6 x 256 227 against
+// 235; back to back the two are level at 1700-2048 rows), FFN1 to 4096 rows
+// (one-slot pass 8.22-8.24 -> 8.11 ms against the register-staged 64x64 at
+// 2049-3072 rows): more workgroups than CUs keep every CU busy.  At 4097-8192 rows alone FFN1 takes 256x192 (19), which
 // covers 8192 rows with one workgroup per CU, and O-proj past pick_deep tile 0.
+// K >= 1024 past pick_deep at 8193-10880 rows: tile 40 in two or more rounds
+// (K = 1536, N = 768 / 1152 / 1536, 8193 rows 43.3 / 44.7 / 67.7 us on tile 32 -> 28.5 /
+// 42.0 / 57.5, 10240 rows 43.9 / 48.4 / 70.7 -> 29.9 / 45.0 / 59.9; level at 12288),
+// but where the second would be a quarter full or less (N = 512, K = 1024, 8193
+// rows 20.1 us, tile 0 17.8).
 // Beside other forwards (shared true: a pool of several slots) every tile was
 // tried for each (shape, M) with the others fixed in the per-batch pass, then
 // the winners confirmed in interleaved repeats: FFN1 takes the 128x128
@@ -1876,10 +1882,10 @@ int pick_plain(int M, int N, int K, bool shared) {
     id = qkv ? 30 : ffn1 ? (shared ? 26 : 19) : wide_k ? 31 : 0;
   else if (M <= 8192)
     id = shared ? (wide_k ? 31 : 30) : qkv || ffn1 ? 19 : wide_k ? 30 : 0;
-  else if (M <= 10880)
-    id = wide_k ? 40 : 30;
   else if (M <= 16384)
-    id = wide_k ? 32 : 30;
+    id = !wide_k ? 30
+         : M <= 10880 && N % 128 == 0 && (long)((M + 127) / 128) * (N / 128) > kCus * 5 / 4 ? 40
+                                                                                            : 32;
   else if (M <= 49152)
     id = wide_k ? 19 : 30;
   else
