@@ -84,17 +84,15 @@ constexpr float kLazy = 8.f;
 template <int NW, int T, int F, bool VL = false>
 __global__ __launch_bounds__(64 * NW, T == 2 || NW > 8 ? 4 : 6) void attention_kernel(
     const f16* __restrict__ qkv, const int32_t* __restrict__ mask, f16* __restrict__ out,
-    int batch, int seq, int heads, float c, const PackedSentence* __restrict__ sents) {
+    int batch, int seq, int heads, float c, const PackedSentence* __restrict__ sents,
+    int last_first) {
   HIP_DYNAMIC_SHARED(f16, smem);
   // (sequence, head) of this workgroup; the heads of a sequence go to one XCD
   // back to back (but where its span ends), so its QKV rows are fetched into
-  // one L2.  Last sequence first: the QKV Linear wrote its rows in ascending
-  // order, and of more than the 256 MB that the memory-side cache holds (302 MB
-  // at 256 x 512) the last ones are still there, where an ascending walk would
-  // evict each row before it is read (bert_embed 256 x 512 4.46 -> 4.37 ms).
+  // one L2.  last_first: the last sequence first (launch_attention).
   const int item = xcd_item(batch, heads);
   if (item < 0) return;
-  const int bq = item / heads, h = item - bq * heads, b = batch - 1 - bq;
+  const int bq = item / heads, h = item - bq * heads, b = last_first ? batch - 1 - bq : bq;
   size_t row0 = (size_t)b * seq;  // first hidden row of the sentence
   if constexpr (VL) {
     const PackedSentence sn = sents[b];
@@ -319,17 +317,23 @@ __global__ __launch_bounds__(64 * NW, T == 2 || NW > 8 ? 4 : 6) void attention_k
 template <int NW, int T, int F, bool VL = false>
 hipError_t launch_attention(const f16* qkv, const int32_t* mask, f16* merged, int batch,
                             int heads, int seq, float c, hipStream_t s,
-                            const PackedSentence* sents = nullptr) {
+                            const PackedSentence* sents, int rows) {
   const int tiles = (seq + 31) / 32;  // for VL: of the longest sentence
   const int staged = !(F & 1) || ((F & 2) && tiles <= NW * T) ? 0 : NW * T;
   static const hipError_t attr = hipFuncSetAttribute(
       reinterpret_cast<const void*>(attention_kernel<NW, T, F, VL>),
       hipFuncAttributeMaxDynamicSharedMemorySize, (int)attn_lds_bytes(kMaxPos, NW * T));
   if (attr != hipSuccess) return attr;
+  // Last sequence first where the QKV rows exceed the memory-side cache: the QKV
+  // Linear wrote them in ascending order, so the last ones are still there, and
+  // an ascending walk would evict each row before it is read (bert_embed 1024 x
+  // 128 4.10 -> 4.00 ms, 512 x 256 4.22 -> 4.13, 256 x 512 4.55 -> 4.51, 224 x 512, 264
+  // MB, 4.14 -> 4.09; level at 192 x 512, 226 MB, padded and packed).
+  const bool last_first = (size_t)rows * 3 * heads * kHeadDim * sizeof(f16) > kMemCache;
   const int grid = xcd_grid(batch, heads);
   hipLaunchKernelGGL((attention_kernel<NW, T, F, VL>), dim3(grid), dim3(64 * NW),
                      attn_lds_bytes(seq, staged), s, qkv, mask, merged, batch, seq, heads, c,
-                     sents);
+                     sents, (int)last_first);
   return hipGetLastError();
 }
 
@@ -353,11 +357,12 @@ hipError_t launch_attention(const f16* qkv, const int32_t* mask, f16* merged, in
 //    two: 160 x 288 47.2 -> 44.9).
 template <bool VL>
 hipError_t attention_any(const f16* qkv, const int32_t* mask, f16* merged, int batch, int heads,
-                         int seq, float scale, hipStream_t s, const PackedSentence* sents) {
+                         int seq, float scale, hipStream_t s, const PackedSentence* sents,
+                         int rows) {
   const float c = scale * 1.4426950408889634f;  // scores * c are base-2 exponents
   const int tiles = (seq + 31) / 32;
 #define BBH_ATT(NW, T, F) \
-  launch_attention<NW, T, F, VL>(qkv, mask, merged, batch, heads, seq, c, s, sents)
+  launch_attention<NW, T, F, VL>(qkv, mask, merged, batch, heads, seq, c, s, sents, rows)
   const int wgs = batch * heads;
   if (tiles >= 16) return BBH_ATT(8, 2, 3);
   if (tiles == 8) return BBH_ATT(4, 2, 3);
@@ -376,13 +381,14 @@ hipError_t attention_any(const f16* qkv, const int32_t* mask, f16* merged, int b
 
 hipError_t attention(const f16* qkv, const int32_t* mask, f16* merged, int batch, int heads,
                      int seq, float scale, hipStream_t s) {
-  return attention_any<false>(qkv, mask, merged, batch, heads, seq, scale, s, nullptr);
+  return attention_any<false>(qkv, mask, merged, batch, heads, seq, scale, s, nullptr,
+                              batch * seq);
 }
 
 hipError_t attention_packed(const f16* qkv, const PackedSentence* sents, int n, f16* merged,
-                            int heads, int max_len, float scale, hipStream_t s) {
+                            int heads, int max_len, int rows, float scale, hipStream_t s) {
   if (n == 0 || max_len == 0) return hipSuccess;
-  return attention_any<true>(qkv, nullptr, merged, n, heads, max_len, scale, s, sents);
+  return attention_any<true>(qkv, nullptr, merged, n, heads, max_len, scale, s, sents, rows);
 }
 
 namespace {

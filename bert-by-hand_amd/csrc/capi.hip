@@ -472,9 +472,10 @@ struct Segment {
   size_t row;
 };
 
-// A packed forward: n sentences (their plan in ws->sents), the longest max_len.
+// A packed forward: n sentences (their plan in ws->sents), the longest max_len,
+// rows tokens in all.
 struct Packed {
-  int n, max_len;
+  int n, max_len, rows;
 };
 
 // out = LN(A . W^T + bias + residual) over 384-wide rows: one kernel where
@@ -516,7 +517,7 @@ bbh_status run_attention(bbh_workspace* ws, const Segment* segs, int n_segs, hip
   if (pk) {
     BBH_TRY(timed_op(t, s, {BBH_OP_ATTENTION, -1, 0, pk->n, pk->max_len, BBH_NUM_HEADS, 0.f}, [&] {
       return check_launch(bbh::attention_packed(ws->qkv, ws->sents, pk->n, ws->ctx, BBH_NUM_HEADS,
-                                                pk->max_len, kScale, s),
+                                                pk->max_len, pk->rows, kScale, s),
                           "attention (packed)");
     }));
   }
@@ -1886,7 +1887,7 @@ bbh_status bbh_embed_packed(bbh_pool* pool, const bbh_model* m, const int32_t* i
             "hipMemcpyAsync(plan)");
     BBH_HIP(hipEventRecord(sl.copied[j], st), "hipEventRecord(plan copied)");
     sl.pending[j] = true;
-    const Packed pk{(int)cnt, max_len};
+    const Packed pk{(int)cnt, max_len, M};
     BBH_TRY(run_encode_packed(w, m, ids, types, pk, M, w->attn_out, st, pool->timer));
     BBH_TRY(timed_op(pool->timer, st, {BBH_OP_POOL, -1, 0, (int)cnt, max_len, 0, 0.f}, [&] {
       return check_launch(bbh::pool_normalize_packed(w->attn_out, w->sents, (int)cnt,

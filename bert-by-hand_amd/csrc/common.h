@@ -22,6 +22,7 @@ constexpr int kFfn = 1536;
 constexpr int kVocab = 30522;
 constexpr int kMaxPos = 512;
 constexpr size_t kLdsMax = 160 * 1024;  // LDS per workgroup on gfx950
+constexpr size_t kMemCache = 256000000;  // bytes of the memory-side cache (Infinity Cache)
 constexpr int kTypes = 2;
 
 // Workgroup b runs on XCD b % 8, each XCD with its own L2 and 32 CUs.

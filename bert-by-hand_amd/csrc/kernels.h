@@ -105,9 +105,10 @@ hipError_t attention(const f16* qkv, const int32_t* mask, f16* merged, int batch
                      int heads, int seq, float scale, hipStream_t s);
 
 // The same over packed sentences (no padding rows, no mask): workgroup (s, h)
-// attends over rows sents[s].row .. + len.  max_len bounds every len.
+// attends over rows sents[s].row .. + len.  max_len bounds every len, rows is
+// their sum.
 hipError_t attention_packed(const f16* qkv, const PackedSentence* sents, int n, f16* merged,
-                            int heads, int max_len, float scale, hipStream_t s);
+                            int heads, int max_len, int rows, float scale, hipStream_t s);
 
 // Reference-shaped attention pieces (unfused): scores, masked softmax, context.
 hipError_t attention_scores(const f16* qkv, f16* scores, int batch, int heads, int seq,
