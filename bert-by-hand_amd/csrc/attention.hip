@@ -90,9 +90,9 @@ __global__ __launch_bounds__(64 * NW, T == 2 || NW > 8 ? 4 : 6) void attention_k
   // (sequence, head) of this workgroup; the heads of a sequence go to one XCD
   // back to back (but where its span ends), so its QKV rows are fetched into
   // one L2.  last_first: the last sequence first (launch_attention).
-  const int item = xcd_item(batch, heads);
-  if (item < 0) return;
-  const int bq = item / heads, h = item - bq * heads, b = last_first ? batch - 1 - bq : bq;
+  int b, h;
+  if (!xcd_item(batch, heads, b, h)) return;
+  if (last_first) b = batch - 1 - b;
   size_t row0 = (size_t)b * seq;  // first hidden row of the sentence
   if constexpr (VL) {
     const PackedSentence sn = sents[b];

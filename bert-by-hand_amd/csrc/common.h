@@ -27,8 +27,8 @@ constexpr int kTypes = 2;
 
 // Workgroup b runs on XCD b % 8, each XCD with its own L2 and 32 CUs.
 // xcd_item deals rows * cols items (row-major) to the XCDs and gives this
-// workgroup's item, or -1.  The items of a row share operands, so they go to
-// one XCD's L2.
+// workgroup's row and column, or false.  The items of a row share operands, so
+// they go to one XCD's L2.
 //  - From kXcdRows rows on, row r goes to XCD r % 8, in order (spans, below,
 //    measured slower there: FFN2 at 46656 rows 97 us against 89).
 //  - Below that, contiguous spans whose lengths differ by at most one item: no
@@ -48,14 +48,26 @@ __host__ __device__ inline int xcd_grid(int rows, int cols) {
   const int n = xcds_for(rows, cols);
   return (rows * cols + n - 1) / n * kXcds;
 }
-__device__ __forceinline__ int xcd_item(int rows, int cols) {
+// One integer division on each way: a workgroup's first load waits for it
+// (bert_encode 21 x 304 394 us with two or three, 391 with one).
+__device__ __forceinline__ bool xcd_item(int rows, int cols, int& row, int& col) {
   const int x = blockIdx.x % kXcds, k = blockIdx.x / kXcds;
   if (rows >= kXcdRows) {
-    const int row = k / cols * kXcds + x;
-    return row < rows ? row * cols + k % cols : -1;
+    const int q = k / cols;
+    row = q * kXcds + x;
+    col = k - q * cols;
+    return row < rows;
   }
-  const int n = xcds_for(rows, cols), q = rows * cols / n, r = rows * cols % n;
-  return x < n && k < q + (x < r ? 1 : 0) ? x * q + min(x, r) + k : -1;
+  if (xcds_for(rows, cols) < kXcds) {
+    row = x;
+    col = k;
+    return row < rows;  // xcd_grid gives k < cols
+  }
+  const int items = rows * cols, q = items / kXcds, r = items % kXcds;
+  const int item = x * q + min(x, r) + k;
+  row = item / cols;
+  col = item - row * cols;
+  return k < q + (x < r ? 1 : 0);
 }
 
 // Lane exchanges without the LDS.  __shfl_xor compiles to ds_bpermute, an

@@ -465,10 +465,7 @@ __device__ __forceinline__ void mainloop_reg(const f16* __restrict__ A,
 
 // Tile coordinates from the workgroup id, XCD-aware (see header).
 __device__ __forceinline__ bool tile_of(int nb, int mb, int& mi, int& ni) {
-  const int t = xcd_item(mb, nb);
-  mi = t / nb;
-  ni = t - mi * nb;
-  return t >= 0;
+  return xcd_item(mb, nb, mi, ni);
 }
 
 // Write ROWS rows of the output tile, staged in LDS as ROWS x OUT_LD fp16,
@@ -986,9 +983,9 @@ __global__ __launch_bounds__(64 * (BM_ / 32 * WN_ + NP_)) void qkv_attention_ker
   using C = typename L::C;
   constexpr int BM = L::BM, KR = L::KR, VLD = L::VLD, NT = L::NT;
   HIP_DYNAMIC_SHARED(f16, smem);
-  const int item = xcd_item((batch + G - 1) / G, kHeads);
-  if (item < 0) return;  // the whole workgroup: no barrier reached
-  const int b0 = item / kHeads * G, h = item % kHeads;
+  int grp, h;
+  if (!xcd_item((batch + G - 1) / G, kHeads, grp, h)) return;  // whole workgroup: no barrier reached
+  const int b0 = grp * G;
   const int gv = min(G, batch - b0), M = batch * seq, m0 = b0 * seq, R = gv * seq;
   const int ntq = (seq + 31) >> 5, KP = ntq * 32;  // query tiles (key chunks) per sentence
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r32 = lane & 31, kh = lane >> 5;
