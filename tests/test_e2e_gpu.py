@@ -599,17 +599,17 @@ def test_embed_packed_edge_cases(torch_cuda, model):
     pool.close()
 
 
-@pytest.mark.parametrize("S", [256, 320, 512])
-def test_embed_packed_long_sentences(torch_cuda, model, S):
-    # Long packed sentences take the other attention shapes (8 query tiles:
-    # 4 wavefronts x 2 tiles; 9-15: 8 x 1 without output staging; 16: 8 x 2),
-    # with sentences of every tile count in one launch.  Bit for bit against
-    # the padded path (both forwards under 8192 rows: separate LayerNorm).
+@pytest.mark.parametrize("S,B", [(256, 16), (320, 16), (512, 16), (320, 110), (512, 300)])
+def test_embed_packed_long_sentences(torch_cuda, model, S, B):
+    # Long packed sentences take the other attention shapes (8 query tiles: 4
+    # wavefronts x 2 tiles; 9-15: 12 x 1, in large batches of 9-11 tiles 8 x 1,
+    # without output staging; 16: 8 x 2), with sentences of every tile count in
+    # one launch.  Bit for bit against the padded path (both forwards under 8192
+    # rows, both between 8193 and 65535, or both above).
     from bbh import engine
 
     torch = torch_cuda
     rng = np.random.default_rng(S)
-    B = 16
     n = rng.integers(0, S + 1, size=B)
     n[:4] = [0, 1, S, 32 * (S // 64) + 1]
     mask = (np.arange(S)[None, :] < n[:, None]).astype(np.int32)

@@ -63,9 +63,8 @@ def test_linear(torch_cuda, M, N, K, gelu):
 def test_linear_rows_identical_across_kernels(torch_cuda, N, gelu):
     # The first rows of a large-M GEMM equal the same rows computed alone:
     # every kernel accumulates in the same k order and rounds the same way.
-    # M = 50000 runs QKV and FFN1 on the weight-resident kernel and N = 384 on
-    # a 128x128 tile; M = 2048 runs all three on 64x64 tiles; M = 3000 runs
-    # N = 384 below and above one workgroup per CU.
+    # M = 50000 runs all three on the weight-resident kernel, M = 2048 on 64x64
+    # tiles; M = 3000 QKV on a 128x128, FFN1 on a 64x64, N = 384 on a 96x64 tile.
     torch = torch_cuda
     from bbh import engine
 
@@ -327,7 +326,7 @@ def test_attention_bits_do_not_depend_on_the_padding(torch_cuda):
     from bbh import engine
 
     rng = np.random.default_rng(7)
-    for n in (16, 45, 100, 130, 250, 300):
+    for n in (32, 45, 100, 130, 250, 300):
         qkv = _h(rng, (2, 512, 1152), 2.0)
         qkv[0, :, 384:768] += (np.arange(512)[:, None] * 0.02).astype(np.float16)
         ref = None
@@ -347,6 +346,44 @@ def test_attention_bits_do_not_depend_on_the_padding(torch_cuda):
             if not two(S):
                 assert np.array_equal(got[:, :n // 32 * 32], ref[:, :n // 32 * 32]), (n, S)
             assert np.abs(got.astype(np.float32) - ref.astype(np.float32)).max() <= 4e-3, (n, S)
+
+
+@pytest.mark.parametrize("B,S", [(107, 288), (110, 352), (107, 368), (172, 496), (256, 512),
+                                 (60, 256), (300, 96)])
+def test_attention_bits_do_not_depend_on_the_batch(torch_cuda, B, S):
+    # From 1281 (sequence, head) pairs on, 9-11 query tiles run on 8 wavefronts
+    # instead of 12; 8 and 16 tiles take one shape in every batch (two tiles a
+    # wavefront).  The rows of a sentence are, bit for bit, those it has in a
+    # batch of three, scores rising along the keys included, and close to fp32.
+    # (256 x 512 also walks the sequences from the last one.)
+    torch = torch_cuda
+    from bbh import engine
+
+    g = torch.Generator(device="cuda").manual_seed(S)
+    qkv = 2.0 * torch.randn((B, S, 1152), device="cuda", generator=g)
+    qkv[:, :, 384:768] += 0.02 * torch.arange(S, device="cuda")[None, :, None]
+    qkv = qkv.half()
+    n = torch.randint(1, S + 1, (B,), device="cuda", generator=g)
+    n[0] = S
+    mask = (torch.arange(S, device="cuda")[None] < n[:, None]).int()
+
+    def attend(rows):
+        out = torch.empty((len(rows) * S, 384), dtype=torch.float16, device="cuda")
+        engine.launch_attention(qkv[rows].reshape(-1, 1152).contiguous(), mask[rows].contiguous(),
+                                out, len(rows), S)
+        return out.view(len(rows), S, 384)
+
+    whole = attend(list(range(B)))
+    few = [0, B // 2, B - 1]
+    part = attend(few)
+    for i, b in enumerate(few):
+        assert torch.equal(part[i], whole[b]), b
+        q, k, v = (qkv[b].float()[:, 384 * j:384 * j + 384].reshape(S, 12, 32).transpose(0, 1)
+                   .contiguous() for j in range(3))
+        p = torch.softmax((q @ k.transpose(1, 2).contiguous()) / 32 ** 0.5
+                          + torch.where(mask[b] != 0, 0.0, float("-inf")), -1)
+        want = (p @ v).transpose(0, 1).reshape(S, 384)
+        assert (whole[b].float() - want).abs().max().item() <= TOL, b
 
 
 def test_unfused_attention_pieces_match_fused(torch_cuda):
