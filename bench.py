@@ -230,22 +230,6 @@ def launch_work(r):
     return flops, byts
 
 
-def qkv_attention_rows(batch, seq, shared=False):
-    """Rows of a qkv_attention_kernel workgroup, the first template argument of
-    its kernel symbol (the launcher's rule): alone the smallest of 64 / 128 /
-    192 / 256 rows that gives at most one workgroup per CU, past that 128 or
-    192, whichever takes fewer rounds of two workgroups a CU times rows;
-    beside other forwards 192 for seq 48, 80 and 96, else 128."""
-    if shared:
-        return 192 if seq in (48, 80, 96) else 128
-    wgs = lambda rows: 12 * -(-batch // (rows // seq))  # noqa: E731
-    for rows in (64, 128, 192, 256):
-        if rows >= seq and wgs(rows) <= 256:
-            return rows
-    cost = lambda rows: -(-wgs(rows) // 512) * rows  # noqa: E731
-    return 128 if cost(128) < cost(192) else 192
-
-
 def kernel_name(engine, op, tile, fused, batch=0, seq=0):
     """(display name, class name as short_kernel() writes it) of a launch record
     of a forward alone; batch, seq: of a fused QKV + attention record (n, k)."""
@@ -255,7 +239,7 @@ def kernel_name(engine, op, tile, fused, batch=0, seq=0):
     if op in row:
         return row[op], row[op]
     if op == "qkv" and fused == 3:
-        name = f"qkv_attention_kernel<{qkv_attention_rows(batch, seq)}>"
+        name = f"qkv_attention_kernel<{engine.qkv_attention_name(batch, seq)}>"
         return name, name
     if fused == 2:  # the LayerNorm carried between the GEMMs as row statistics
         epi = {"qkv": "4 (carried LayerNorm in)", "ffn1_gelu": "5 (carried LayerNorm in+GELU)"}.get(
@@ -266,23 +250,6 @@ def kernel_name(engine, op, tile, fused, batch=0, seq=0):
     if tname.startswith("WRes"):
         return f"gemm_wres_kernel<{epi}>", f"gemm_wres_kernel<{epi[0]}>"
     return f"gemm_kernel<{tname}, {epi}>", f"gemm_kernel<{tname}, {epi[0]}>"
-
-
-def gemm_grid_items(tile_name, M, N):
-    """Work-items of a tiled-GEMM launch (the launcher's grid: whole rows of tiles
-    dealt to 8 XCDs from 96 rows on, below that the tiles in even spans, below 8
-    rows of at most 32 tiles one XCD a row; 64 threads for each computing and each copying wavefront), as rocprofv3
-    reports Grid_Size; None for other kernels."""
-    import re
-
-    m = re.match(r"Cfg<(\d+),(\d+),(\d+),(\d+),(\d+),(-?\d+),", tile_name)
-    if not m:
-        return None
-    bm, bn, wm, wn, _, pd = (int(x) for x in m.groups())
-    rows, cols = -(-M // bm), N // bn
-    xcds = rows if rows < 8 and cols <= 32 else 8
-    per_xcd = -(-rows // 8) * cols if rows >= 96 else -(-rows * cols // xcds)
-    return per_xcd * 8 * 64 * (wm * wn + (-pd % 256 // 16 if pd < 0 else 0))
 
 
 def classify(engine, recs, steps):
@@ -304,7 +271,7 @@ def classify(engine, recs, steps):
         avg_s = c["ms"] / c["n"] / 1e3
         name, cls = kernel_name(engine, op, tile, fused, batch, seq)
         n_out = {"qkv": 1152, "ffn1_gelu": 1536}.get(op, 384)
-        grid = gemm_grid_items(engine.gemm_tile_name(tile), m, n_out) if tile >= 0 else None
+        grid = (engine.gemm_grid(tile, m, n_out) or None) if tile >= 0 else None
         rows.append({"kernel": name, "class": cls, "op": op, "m": m, "grid_items": grid,
                      "launches_per_step": round(c["n"] / steps, 2),
                      "avg_launch_us": round(avg_s * 1e6, 2),
@@ -331,9 +298,10 @@ def short_kernel(name):
     m = re.search(r"gemm_wres_kernel(?:<|ILi)(\d)", n)
     if m:
         return f"gemm_wres_kernel<{m.group(1)}>"
-    m = re.search(r"qkv_attention_kernel(?:<|ILi)(\d+)", n)
+    m = (re.search(r"qkv_attention_kernel<(\d+),(\d+),(\d+),(\d+)>", n) or
+         re.search(r"qkv_attention_kernelILi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)E", n))
     if m:
-        return f"qkv_attention_kernel<{m.group(1)}>"
+        return f"qkv_attention_kernel<{','.join(m.groups())}>"
     m = (re.search(r"attention_kernel<(\d+),(\d+),(\d+),(\w+)>", n) or
          re.search(r"attention_kernelILi(\d+)ELi(\d+)ELi(\d+)ELb(\d)E", n))
     if m:
@@ -475,25 +443,28 @@ def trace_summary(trace, stream):
     return "\n".join(lines)
 
 
-# (tile id, M, N, K, epilogue): a shape at which bbh_linear (epilogue "bias" /
-# "gelu") or bbh_linear_residual_layernorm ("ln") launches that tile, for the
-# tile configurations the forwards pick (1 is picked only beside other
-# forwards: the per-batch pass on several slots).
-TILE_SHAPES = [(0, 1024, 1536, 384, "gelu"), (26, 1024, 384, 384, "bias"),
-               (34, 3072, 384, 1536, "bias"),
-               (30, 1024, 1152, 384, "bias"), (31, 8192, 384, 1536, "bias"),
-               (32, 16384, 384, 1536, "bias"), (19, 32768, 384, 1536, "bias"),
-               (14, 16384, 384, 1536, "ln"),
-               (28, 32768, 384, 384, "ln"), (18, 32768, 384, 1536, "ln"),
-               (33, 32768, 1152, 384, "bias")]
+# (M, N, K, epilogue): a shape at which bbh_linear (epilogue "bias" / "gelu") or
+# bbh_linear_residual_layernorm ("ln") launches each tile configuration that
+# the forwards pick alone, in the order of their ids (26 and 31 are picked only
+# beside other forwards: the per-batch pass on several slots).
+TILE_SHAPES = [(4096, 1536, 384, "gelu"), (16384, 384, 1536, "ln"), (32768, 384, 1536, "ln"),
+               (8192, 1536, 384, "gelu"), (32768, 384, 384, "ln"), (3072, 1152, 384, "bias"),
+               (16384, 384, 1536, "bias"), (32768, 1152, 384, "bias"), (256, 384, 1536, "bias"),
+               (2048, 384, 1536, "bias"), (3072, 384, 1536, "bias"), (4096, 384, 1536, "bias"),
+               (6144, 384, 1536, "bias"), (8192, 384, 1536, "bias"), (1024, 1536, 384, "gelu")]
+# (batch, seq): the attention kernel's workgroup shapes
+ATTENTION_SHAPES = [(64, 144), (64, 256), (21, 304), (160, 288), (40, 384), (256, 512)]
 
 
-def run_tiles(torch, engine, steps, warmup):
-    """Each TILE_SHAPES launch, timed alone: {"tile M N K epi": us}."""
+def run_tiles(torch, engine, model, steps, warmup):
+    """Each TILE_SHAPES launch, timed alone: {"tile M N K epi": us}; then the FFN
+    block at 12288 rows (FFN2 from the model's sliced weights, tile 42) and the
+    attention kernel at ATTENTION_SHAPES."""
     gen = torch.Generator(device="cuda").manual_seed(3)
     h = lambda *shape: (torch.randn(*shape, device="cuda", generator=gen) * 0.5).half()  # noqa: E731
     out = {}
-    for tile, M, N, K, epi in TILE_SHAPES:
+    for M, N, K, epi in TILE_SHAPES:
+        tile = engine.linear_tile(M, N, K, epi == "ln")
         A, W, b = h(M, K), h(N, K), h(N)
         C = torch.empty((M, N), dtype=torch.float16, device="cuda")
         if epi == "ln":
@@ -502,6 +473,15 @@ def run_tiles(torch, engine, steps, warmup):
         else:
             fn = lambda: engine.launch_matmul(A, W, C, M, N, K, bias=b, gelu=epi == "gelu")  # noqa: E731
         out[f"{tile} {M}x{N}x{K} {epi}"] = round(timed(torch, fn, steps, warmup) * 1e3, 2)
+    ws, x, y = engine.Workspace(96, 128), h(12288, 384), h(12288, 384)
+    fn = lambda: engine.ffn_block(ws, model, 0, x, y, 96, 128)  # noqa: E731
+    out["ffn_block 96x128"] = round(timed(torch, fn, steps, warmup) * 1e3, 2)
+    ws.close()
+    for B, S in ATTENTION_SHAPES:
+        qkv, ctx = h(B * S, 1152), h(B * S, 384)
+        mask = torch.ones((B, S), dtype=torch.int32, device="cuda")
+        fn = lambda: engine.launch_attention(qkv, mask, ctx, B, S)  # noqa: E731
+        out[f"attention {B}x{S}"] = round(timed(torch, fn, steps, warmup) * 1e3, 2)
     return out
 
 
@@ -645,7 +625,7 @@ def main():
               flush=True)
         return
     if args.only == "tiles":  # one kernel-level launch per tile configuration the product picks
-        print(json.dumps(run_tiles(torch, engine, args.steps, args.warmup)), flush=True)
+        print(json.dumps(run_tiles(torch, engine, model, args.steps, args.warmup)), flush=True)
         model.close()
         return
     if args.only in ("packed", "merged"):  # the varlen mix through bbh_embed_packed / _batches

@@ -112,6 +112,13 @@ SIGNATURES = {
                              c_void_p, c_void_p]),
 }
 
+# Exported for profile tables only: what the launchers choose.
+QUERIES = {
+    "bbh_linear_tile": (c_int, [c_int, c_int, c_int, c_int]),
+    "bbh_gemm_grid": (ctypes.c_int64, [c_int, c_int, c_int]),
+    "bbh_qkv_attention_name": (c_char_p, [c_int, c_int, c_int]),
+}
+
 STATUS = {
     0: "BBH_OK", 1: "BBH_ERR_INVALID_ARG", 2: "BBH_ERR_SEQ_ALIGN", 3: "BBH_ERR_CAPACITY",
     4: "BBH_ERR_IO", 5: "BBH_ERR_HIP", 6: "BBH_ERR_OOM", 7: "BBH_ERR_UNSUPPORTED",
@@ -142,7 +149,7 @@ def lib():
         import torch  # noqa: F401
 
         L = ctypes.CDLL(LIB_PATH)
-        for name, (res, args) in SIGNATURES.items():
+        for name, (res, args) in {**SIGNATURES, **QUERIES}.items():
             fn = getattr(L, name)
             fn.restype = res
             fn.argtypes = args

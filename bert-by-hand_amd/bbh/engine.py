@@ -499,4 +499,19 @@ def gemm_tile_name(tile: int) -> str:
     return capi.lib().bbh_gemm_tile_name(tile).decode()
 
 
+def linear_tile(M: int, N: int, K: int, residual_ln: bool = False) -> int:
+    """Tile id of launch_matmul (launch_linear_residual_layernorm) at a shape."""
+    return capi.lib().bbh_linear_tile(M, N, K, int(residual_ln))
+
+
+def gemm_grid(tile: int, M: int, N: int) -> int:
+    """Work-items of a launch of a tile, 0 for other kernels."""
+    return capi.lib().bbh_gemm_grid(tile, M, N)
+
+
+def qkv_attention_name(batch: int, seq: int, shared: bool = False) -> str:
+    """Template arguments of the QKV + attention kernel of a padded forward."""
+    return capi.lib().bbh_qkv_attention_name(batch, seq, int(shared)).decode()
+
+
 BBHError = capi.BBHError

@@ -1944,6 +1944,26 @@ bbh_status bbh_pool_timing_read(bbh_pool* pool, bbh_launch_time* out, int max, i
 
 const char* bbh_gemm_tile_name(int tile) { return bbh::gemm_tile_name(tile); }
 
+// Queries for profile tables, not part of the interface (host only): what the
+// launchers choose.  The tile of bbh_linear (residual_ln 0) or
+// bbh_linear_residual_layernorm (1) at 16-byte aligned operands; the work-items
+// of a launch of `tile`, as a profiler reports them (0: not a tiled GEMM); the
+// template arguments of the QKV + attention kernel (launch records with
+// fused_ln 3) of a forward alone or beside others (null: sizes it does not take).
+int bbh_linear_tile(int M, int N, int K, int residual_ln) {
+  if (M < 1 || N < 1 || K < 1) return -1;
+  bool fused;
+  return residual_ln ? bbh::gemm_residual_ln_tile(M, K, &fused) : bbh::gemm_tile(M, N, K);
+}
+
+int64_t bbh_gemm_grid(int tile, int M, int N) {
+  return M < 1 || N < 1 ? 0 : bbh::gemm_grid(tile, M, N);
+}
+
+const char* bbh_qkv_attention_name(int batch, int seq, int shared) {
+  return bbh::qkv_attention_name(batch, seq, shared != 0);
+}
+
 static bbh_status check_layer(const bbh_workspace* ws, const bbh_model* m, int layer,
                               const void* hidden, const void* out, int batch, int seq) {
   if (!ws || !m || !hidden || !out) return fail(BBH_ERR_INVALID_ARG, "null argument");

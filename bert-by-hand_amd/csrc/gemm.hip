@@ -1923,6 +1923,19 @@ int gemm_residual_ln_tile(int M, int K, bool* fused_ln, bool shared, bool sliced
   return M <= 16384 ? 14 : K >= 1024 ? 18 : 28;
 }
 
+int64_t gemm_grid(int tile, int M, int N) {
+#define BBH_GRID(ID, BM, BN, WM, WN, SA, PD, SW)                              \
+  case ID:                                                                    \
+    return (int64_t)xcd_grid((M + BM - 1) / BM, N / BN) * Cfg<BM, BN, WM, WN, SA, PD, SW>::THREADS;
+  switch (tile) {
+    BBH_TILES(BBH_GRID)
+    BBH_SLICED(BBH_GRID)
+    BBH_TUNING_TILES(BBH_GRID)
+  }
+#undef BBH_GRID
+  return 0;
+}
+
 const char* gemm_tile_name(int tile) {
   if (tile == kTiles) return "WRes<12x32,384>";
   const char* n = tile_name(tile);
@@ -2010,10 +2023,18 @@ hipError_t launch_qkv_attention(const f16* X, const f16* Wp, const float* fs, co
   return hipGetLastError();
 }
 
-// Rows of a workgroup (whole sentences).  Alone, where one workgroup per CU
-// covers the batch: the smallest of 64 / 128 / 192 / 256 rows that gives at
-// most kCus workgroups, with rings 3-4 slices deep (128 and 192 rows: negative,
-// their one-per-CU form).  Past that two workgroups a CU with rings of two
+// The workgroup shapes: X(id, rows, wavefronts across Q|K|V, ring slices, copying
+// wavefronts).
+#define BBH_QA_SHAPES(X) \
+  X(0, 64, 3, 4, 2)      \
+  X(1, 128, 3, 3, 4)     \
+  X(2, 192, 1, 3, 4)     \
+  X(3, 256, 1, 3, 4)     \
+  X(4, 128, 1, 2, 2)     \
+  X(5, 192, 1, 2, 2)
+// Id of the shape, its rows being whole sentences.  Alone, where one workgroup
+// per CU covers the batch: the smallest of 64 / 128 / 192 / 256 rows that gives at
+// most kCus workgroups, with rings 3-4 slices deep.  Past that two workgroups a CU with rings of two
 // slices, 128 or 192 rows, whichever takes fewer rounds times rows.  Beside
 // other forwards (shared) always the latter, 192 rows where 128 would leave
 // a quarter or more of the tile idle (seq 48, 80, 96): deep rings would hold
@@ -2024,13 +2045,23 @@ hipError_t launch_qkv_attention(const f16* X, const f16* Wp, const float* fs, co
 // 9.0 -> 7.1, 64 x 48 10.1 -> 8.8, 64 x 64 10.8 -> 9.4, 100 x 48 14.1 -> 10.2,
 // 32 x 128 11.7 -> 10.3; two a CU: 64 x 80 14.4 -> 12.9, 64 x 128 20.8 -> 18.1,
 // 500 x 16 17.2 -> 12.7.
-int qkv_attention_rows(int batch, int seq, bool shared) {
-  if (shared) return seq == 48 || seq == 80 || seq == 96 ? 192 : 128;
+int qkv_attention_shape(int batch, int seq, bool shared) {
+  if (shared) return seq == 48 || seq == 80 || seq == 96 ? 5 : 4;
   auto groups = [&](int rows) { return (batch + rows / seq - 1) / (rows / seq); };
-  for (int rows : {64, 128, 192, 256})
-    if (rows >= seq && kHeads * groups(rows) <= kCus) return rows == 128 || rows == 192 ? -rows : rows;
+  for (int i = 0; i < 4; ++i)
+    if (64 * (i + 1) >= seq && kHeads * groups(64 * (i + 1)) <= kCus) return i;
   auto cost = [&](int rows) { return (kHeads * groups(rows) + 2 * kCus - 1) / (2 * kCus) * rows; };
-  return cost(128) < cost(192) ? 128 : 192;
+  return cost(128) < cost(192) ? 4 : 5;
+}
+
+const char* qkv_attention_name(int batch, int seq, bool shared) {
+  if (!qkv_attention_ok(batch, seq)) return nullptr;
+#define BBH_QA_NAME(ID, ROWS, WN, R, NP) \
+  case ID:                               \
+    return #ROWS "," #WN "," #R "," #NP;
+  switch (qkv_attention_shape(batch, seq, shared)) { BBH_QA_SHAPES(BBH_QA_NAME) }
+#undef BBH_QA_NAME
+  return nullptr;
 }
 
 bool qkv_attention_ok(int batch, int seq) {
@@ -2044,17 +2075,13 @@ hipError_t qkv_attention(const f16* X, const f16* Wp, const float* fs, const flo
                        (((uintptr_t)cy.st_in) & 15) == 0;
   if (!qkv_attention_ok(batch, seq) || !fc || !mask || !aligned) return hipErrorInvalidValue;
   const float c = scale * 1.4426950408889634f;  // scores * c are base-2 exponents
-#define BBH_QA(...) \
-  launch_qkv_attention<__VA_ARGS__>(X, Wp, fs, fc, cy, mask, ctx, batch, seq, c, eps, s)
-  switch (qkv_attention_rows(batch, seq, shared)) {
-    case 64: return BBH_QA(64, 3, 4, 2);
-    case -128: return BBH_QA(128, 3, 3, 4);
-    case -192: return BBH_QA(192, 1, 3, 4);
-    case 256: return BBH_QA(256, 1, 3, 4);
-    case 192: return BBH_QA(192, 1, 2, 2);
-    default: return BBH_QA(128, 1, 2, 2);
-  }
+#define BBH_QA(ID, ROWS, WN, R, NP)                                                            \
+  case ID:                                                                                     \
+    return launch_qkv_attention<ROWS, WN, R, NP>(X, Wp, fs, fc, cy, mask, ctx, batch, seq, c, eps, \
+                                                 s);
+  switch (qkv_attention_shape(batch, seq, shared)) { BBH_QA_SHAPES(BBH_QA) }
 #undef BBH_QA
+  return hipErrorInvalidValue;
 }
 
 hipError_t gemm_fold(const f16* A, const f16* W, const LnCarry& cy, f16* C, int M, int N, int K,

@@ -75,6 +75,10 @@ hipError_t qkv_attention(const f16* X, const f16* Wp, const float* fs, const flo
 int gemm_tile(int M, int N, int K, bool shared = false);
 int gemm_residual_ln_tile(int M, int K, bool* fused_ln, bool shared = false, bool sliced = false);
 const char* gemm_tile_name(int tile);
+// Work-items of a launch of a tile (0: not a tile of the table), and the
+// template arguments of the kernel that qkv_attention() launches (null: none).
+int64_t gemm_grid(int tile, int M, int N);
+const char* qkv_attention_name(int batch, int seq, bool shared);
 
 // y(M,384) = LN(A(M,K) . W(384,K)^T + bias + residual) * gamma + beta.
 // y may alias residual.  K % 64 == 0.  W_slices: W again, where the caller

@@ -312,7 +312,7 @@ typedef struct bbh_launch_time {
 } bbh_launch_time;
 bbh_status bbh_pool_timing(bbh_pool *pool, int capacity);
 bbh_status bbh_pool_timing_read(bbh_pool *pool, bbh_launch_time *out, int max, int *count);
-/* "Cfg<BM,BN,WM,WN,SA,PD>" of a GEMM tile configuration, the template
+/* "Cfg<BM,BN,WM,WN,SA,PD,SW>" of a GEMM tile configuration, the template
  * argument in the kernel symbol gemm_kernel<Cfg<...>, epilogue>. */
 const char *bbh_gemm_tile_name(int tile);
 

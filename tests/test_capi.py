@@ -3,6 +3,7 @@ header declares, and rejects bad arguments before touching the device.  No
 compute entry point is called without a GPU."""
 
 import ctypes
+import importlib.util
 import os
 import re
 
@@ -169,6 +170,39 @@ def test_tile_names_and_timing_arguments():
     cnt = ctypes.c_int(7)
     assert L.bbh_pool_timing(None, 16) == 1
     assert L.bbh_pool_timing_read(None, None, 0, ctypes.byref(cnt)) == 1
+
+
+def test_launcher_queries():
+    L = _lib()
+    # alone, one workgroup per CU: the smallest of 64 / 128 / 192 / 256 rows in at
+    # most 256 workgroups of whole sentences; past that two a CU; beside others
+    # always those
+    name = lambda *a: L.bbh_qkv_attention_name(*a).decode()  # noqa: E731
+    assert name(1, 16, 0) == name(84, 16, 0) == name(21, 64, 0) == "64,3,4,2"
+    assert name(85, 16, 0) == name(64, 32, 0) == name(21, 128, 0) == "128,3,3,4"
+    assert name(64, 48, 0) == name(84, 48, 0) == name(42, 80, 0) == "192,1,3,4"
+    assert name(85, 48, 0) == name(43, 80, 0) == name(64, 64, 0) == "256,1,3,4"
+    assert name(64, 128, 0) == name(64, 32, 1) == name(1, 112, 1) == "128,1,2,2"
+    assert name(64, 96, 0) == name(64, 48, 1) == name(1, 80, 1) == "192,1,2,2"
+    for B, S in ((0, 16), (1, 144), (1, 20), (65, 128)):
+        assert L.bbh_qkv_attention_name(B, S, 0) is None
+    # work-items: tiles dealt to 8 XCDs, 64 for each wavefront that computes or copies
+    assert L.bbh_gemm_grid(30, 3072, 1152) == 24 * 9 * 512
+    assert L.bbh_gemm_grid(36, 1300, 384) == 128 * 512  # 21 x 6 tiles in spans of 16
+    assert L.bbh_gemm_grid(40, 128 * 97, 384) == 104 * 3 * 512  # whole rows of tiles
+    assert L.bbh_gemm_grid(35, 16, 1536) == 24 * 8 * 384  # one XCD
+    assert L.bbh_gemm_grid(33, 8193, 384) == 0 and L.bbh_gemm_grid(-1, 16, 384) == 0
+    # every tile configuration of the forwards alone has a shape in bench.py's table
+    spec = importlib.util.spec_from_file_location("bench", os.path.join(ROOT, "bench.py"))
+    bench = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(bench)
+    tiles = [L.bbh_linear_tile(M, N, K, epi == "ln") for M, N, K, epi in bench.TILE_SHAPES]
+    assert tiles == [0, 14, 18, 19, 28, 30, 32, 33, 35, 36, 37, 38, 39, 40, 41]
+    assert L.bbh_linear_tile(5, 20, 384, 0) == -1  # the general kernel
+    # weight-resident kernel: last rows before it and first rows on it
+    for N, M in ((384, 21760), (768, 10880), (1152, 10880), (1536, 8192)):
+        assert L.bbh_linear_tile(M, N, 384, 0) != 33 and L.bbh_linear_tile(M + 1, N, 384, 0) == 33
+    assert L.bbh_linear_tile(65535, 384, 384, 1) == 28 and L.bbh_linear_tile(65536, 384, 384, 1) == 33
 
 
 def test_graph_entry_points_validate_before_touching_hip():
