@@ -12,17 +12,22 @@
 // D(n, m) = W . A^T: lane l then holds, per 32x32 block, four runs of four
 // consecutive output columns n of one row m.
 //
-// Operand pipeline: a workgroup of 4 wavefronts owns a BM x BN output tile
-// and walks K in 64-wide slices.  Slices are copied global -> LDS with
-// global_load_lds_dwordx4 (16 bytes per lane, no register staging) into two
-// rings: the activations A, streamed from HBM, run SA-1 slices ahead (their
-// HBM latency is what a single shared ring exposes), the weights W, resident
-// in L2, SW-1 slices ahead (SW = 2 in every configuration in the table: deeper
-// W rings measured no faster); one barrier per slice.  The other pipeline
-// stages PD slices per thread in VGPRs and double-buffers one LDS tile.  Within a slice, row r is
-// 128 bytes = 8 chunks of 16 bytes and logical chunk c sits in slot
-// c ^ ((r >> 1) & 7): the 16 rows one MFMA operand fetch touches per LDS cycle
-// then hit 16 distinct bank groups.
+// Operand pipelines: a workgroup owns a BM x BN output tile and walks K in
+// slices, 64 wide but in tile 42 (32).  Three loops, by tile:
+//  - mainloop: slices are copied global -> LDS with buffer loads to LDS (16
+//    bytes per lane, no register staging) into two rings by the wavefronts that
+//    compute: the activations A, streamed from HBM, run SA-1 slices ahead
+//    (their HBM latency is what a single shared ring exposes), the weights W,
+//    resident in L2, SW-1 slices ahead (SW = 2: deeper W rings measured no
+//    faster here); one barrier per slice.
+//  - mainloop_reg: PD slices per thread in VGPRs and one double-buffered LDS
+//    tile.
+//  - mainloop_deep: one ring of whole slices, filled by wavefronts that only
+//    copy (or, without any, by those that compute), for tiles that have a CU to
+//    themselves.
+// Within a 64-wide slice, row r is 128 bytes = 8 chunks of 16 bytes and logical
+// chunk c sits in slot c ^ ((r >> 1) & 7): the 16 rows one MFMA operand fetch
+// touches per LDS cycle then hit 16 distinct bank groups.
 //
 // Tile order is XCD-aware: workgroup b runs on XCD b % 8, and the N-tiles of
 // one M-tile are given to consecutive workgroups of the same XCD so the A
@@ -1657,10 +1662,10 @@ hipError_t launch(const f16* A, const f16* W, const f16* bias, const f16* residu
   }
 }
 
-// Tile configurations (BM, BN, wavefronts M x N, A-ring depth), by id; the K
-// slice is 64 wide and the W ring 2 deep but in tiles 35-42.  The product build holds
-// the configurations pick_plain and gemm_residual_ln_tile choose; the others
-// of the sweep that chose them are compiled only with -DBBH_TUNING.
+// Tile configurations (BM, BN, wavefronts M x N, A-ring depth), by id.  The
+// product build holds the configurations pick_plain and gemm_residual_ln_tile
+// choose; the others of the sweep that chose them are compiled only with
+// -DBBH_TUNING.
 //   id  tile      wave tile  SA   LDS
 //    0  64x64     32x32      4    48 KB
 //   14  64x384    64x96      2   112 KB   (owns whole 384-wide rows)
@@ -1673,8 +1678,8 @@ hipError_t launch(const f16* A, const f16* W, const f16* bias, const f16* residu
 //   30  128x128   64x32 (8w) PD 2   64 KB
 //   31  128x128   32x64 (8w) PD 2   64 KB
 //   32  128x192   32x96 (8w) PD 2   80 KB
-//   one workgroup per CU, A and W in one ring of SA slices (mainloop_deep),
-//   NP copying wavefronts:
+//   A and W in one ring of SA slices (mainloop_deep), NP copying wavefronts; one
+//   workgroup per CU, but two of 35, 37 and 41 fit:
 //   35  32x64     32x32 (2w) 6     72 KB   NP 4, two slices per barrier
 //   36  64x64     32x32      6     96 KB   NP 4, two slices per barrier
 //   37  96x64     32x32 (6w) 4     80 KB   NP 4
@@ -1805,34 +1810,34 @@ const char* tile_name(int id) {
 // length buckets) the best tile depends on whether other forwards share the
 // CUs.
 // Alone (shared false: bbh_embed, a one-slot pool), pick_deep's tiles first;
-// past them, from sweeps with one GEMM's tile changed at a time: QKV runs the
-// 64x64 copy-ring tile (0) up to 2048 rows (inside bert_embed 4 x 512 304 us
-// against 307 on tile 30, and below, on pick_deep's tiles, 6 x 256 227 against
-// 235; back to back the two are level at 1700-2048 rows), FFN1 to 4096 rows
-// (one-slot pass 8.22-8.24 -> 8.11 ms against the register-staged 64x64 at
-// 2049-3072 rows): more workgroups than CUs keep every CU busy.  At 4097-8192 rows alone FFN1 takes 256x192 (19), which
-// covers 8192 rows with one workgroup per CU, and O-proj past pick_deep tile 0.
-// K >= 1024 past pick_deep at 8193-10880 rows: tile 40 in two or more rounds
-// (K = 1536, N = 768 / 1152 / 1536, 8193 rows 43.3 / 44.7 / 67.7 us on tile 32 -> 28.5 /
-// 42.0 / 57.5, 10240 rows 43.9 / 48.4 / 70.7 -> 29.9 / 45.0 / 59.9; level at 12288),
-// but where the second would be a quarter full or less (N = 512, K = 1024, 8193
-// rows 20.1 us, tile 0 17.8).
+// past them, from sweeps with one GEMM's tile changed at a time:
+//  - QKV: the 64x64 copy-ring tile (0) up to 2048 rows (inside bert_embed 4 x 512
+//    304 us against 307 on tile 30, and below, on pick_deep's tiles, 6 x 256 227
+//    against 235; back to back the two are level at 1700-2048 rows).
+//  - FFN1: tile 0 to 4096 rows (one-slot pass 8.22-8.24 -> 8.11 ms against the
+//    register-staged 64x64 at 2049-3072 rows): more workgroups than CUs keep
+//    every CU busy.  At 4097-8192 rows 256x192 (19), which covers 8192 rows with
+//    one workgroup per CU.
+//  - O-proj: tile 0.
+//  - K >= 1024 at 8193-10880 rows: tile 40 in two or more rounds (K = 1536, N =
+//    768 / 1152 / 1536, 8193 rows 43.3 / 44.7 / 67.7 us on tile 32 -> 28.5 / 42.0 /
+//    57.5, 10240 rows 43.9 / 48.4 / 70.7 -> 29.9 / 45.0 / 59.9; level at 12288), but
+//    where the second would be a quarter full or less (N = 512, K = 1024, 8193
+//    rows 20.1 us, tile 0 17.8).
 // Beside other forwards (shared true: a pool of several slots) every tile was
-// tried for each (shape, M) with the others fixed in the per-batch pass, then
-// the winners confirmed in interleaved repeats: FFN1 takes the 128x128
-// register-staged tile (30) from 1025 rows and FFN2 the 64x128 copy-ring tile
-// (1) from 2049 rows, 391K -> 409K sentences/s for the pass on three streams.
-// With the LayerNorms carried as row statistics (the epilogues heavier), a
-// sweep on four slots moved O-proj to tile 1 as well and QKV to tile 30 up to
-// 4096 rows: pass 4.144-4.160 -> 4.064-4.095 ms in four interleaved repeats;
-// with QKV inside the attention kernel, O-proj to the 128x128 tile (30):
-// 4.117-4.127 -> 4.092-4.104 ms; FFN2 on tile 1 and O-proj on tile 30 from
-// 1025 rows as well (3.708 -> 3.668 ms, then 3.845-3.857 -> 3.828-3.843 ms,
-// four repeats each; alone they are slower there).  With copying wavefronts
-// FFN2 takes tile 40 and O-proj tile 41 from 1025 rows (pass 3.933 -> 3.877 ->
-// 3.864 ms; the tiles with 96 KB and more of LDS, 36-39, +2.7 to +5.5%).
-// There the other forwards fill the CUs, and fewer, larger tiles move fewer
-// bytes L2 -> CU per FLOP.
+// tried for each (shape, M) with the others fixed in the four-slot pass over
+// per-length batches, then the winners confirmed in interleaved repeats: FFN1
+// and, where attention does not compute it, QKV take the 128x128 register-staged
+// tile (30) from 1025 rows, FFN2 the 128x128 deep ring with copying wavefronts
+// (40), O-proj the 64x128 deep ring without (41): pass 3.76 ms with FFN2 on the
+// 64x128 copy ring and O-proj on tile 30 -> 3.74 ms, two interleaved repeats; the
+// tiles 36-39 cost 2.7 to 5.5% there.  The other forwards fill the CUs, and
+// fewer, larger tiles move fewer bytes L2 -> CU per FLOP.
+// A forward on one of several streams that a caller drives without a pool counts
+// as alone: four of 64 x 32 on four streams take 107 us each against 102 with the
+// tiles of the pool, two on two 119 against 128; 64 x 16 64 against 73, 64 x 64 181
+// against 195, 64 x 128 339 against 345 on four.
+//
 // Alone, where one workgroup per CU covers the output (kCus CUs): the smallest
 // of the mainloop_deep tiles that needs at most kCus workgroups.  Such a
 // GEMM is bound by one workgroup's walk over K, which a smaller tile
