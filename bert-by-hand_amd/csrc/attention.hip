@@ -340,21 +340,25 @@ hipError_t launch_attention(const f16* qkv, const int32_t* mask, f16* merged, in
 // Workgroup shape by query-tile count (tiles = ceil(seq / 32); for packed
 // sentences of the longest one).
 //  - 2-4 tiles: 4 wavefronts of one tile each, output staged through the K/V
-//    area (266 x 96 21.2 -> 17.6 us, 600 x 64 23.6 -> 22.1 against one wavefront
-//    a tile).  Packed sentences of up to 3 tiles: 2 wavefronts, for most
-//    sentences are much shorter than the longest.
+//    area.  More wavefronts than tiles still help to stage K and V, but at two
+//    tiles only while all workgroups run at once (six a CU: 1536): 64 x 48 / 128 x
+//    64 4.8 / 6.6 us on 2 wavefronts, 4.7 / 6.4 on 4; 130 x 48 / 171 x 64 6.5 / 8.3
+//    against 7.2 / 8.9.  At three tiles 4 in every batch (309 x 80 23.0 -> 18.8).
+//    Packed sentences of up to 3 tiles: 2 wavefronts, for most sentences are much
+//    shorter than the longest.
 //  - 8 and 16 tiles: 4 and 8 wavefronts of two tiles, output staged.  The two
 //    tiles of a wavefront are rescaled together, which shows in the last bits,
 //    so these counts take this shape in every batch (one tile a wavefront: 512 x
 //    256 129 us against 122 here, 128 x 512 96 against 94, but 64 x 256 20.7
 //    against 21.2).
 //  - Else 5-7 tiles: 8 wavefronts, 9-15: 12, one tile at a time and stored
-//    straight from the accumulators: more wavefronts than tiles still help to
-//    stage K and V, and more of them hide the exp and MFMA latencies than 4 or
-//    8 (64 x 144 / 192 11.2 / 13.7 -> 9.0 / 12.5 us, 21 x 304 12.5 -> 11.3, 80 x
-//    288 / 480 28.0 / 54.9 -> 27.1 / 52.3).  Where a CU's share of workgroups
-//    fills it anyway, 9-11 tiles on 8 wavefronts (three workgroups a CU against
-//    two: 160 x 288 47.2 -> 44.9).
+//    straight from the accumulators: more wavefronts than tiles help here, too,
+//    and more of them hide the exp and MFMA latencies than 4 or 8 (64 x 144 / 192
+//    11.2 / 13.7 -> 9.0 / 12.5 us, 21 x 304 12.5 -> 11.3, 80 x 288 / 480 28.0 / 54.9 ->
+//    27.1 / 52.3).  But 9-11 tiles on 8 wavefronts where a CU's share of workgroups
+//    fills it anyway (160 x 288 47.2 -> 44.9), and 9-10 where that saves a round,
+//    three workgroups a CU against two (43 x 288 / 320 20.8 / 23.7 -> 19.2 / 22.6, 106 x
+//    288 37.1 -> 35.4; 65 x 288, two rounds of either, 27.2 on 12, 27.6 on 8).
 template <bool VL>
 hipError_t attention_any(const f16* qkv, const int32_t* mask, f16* merged, int batch, int heads,
                          int seq, float scale, hipStream_t s, const PackedSentence* sents,
@@ -366,12 +370,14 @@ hipError_t attention_any(const f16* qkv, const int32_t* mask, f16* merged, int b
   const int wgs = batch * heads;
   if (tiles >= 16) return BBH_ATT(8, 2, 3);
   if (tiles == 8) return BBH_ATT(4, 2, 3);
-  if (tiles > (wgs > 1280 ? 11 : 8)) return BBH_ATT(12, 1, 0);
+  auto rounds = [&](int per_cu) { return (wgs + 256 * per_cu - 1) / (256 * per_cu); };
+  const bool eight = wgs > 1280 ? tiles <= 11 : tiles <= 10 && rounds(3) < rounds(2);
+  if (tiles > 8 && !eight) return BBH_ATT(12, 1, 0);
   if (tiles > 4) return BBH_ATT(8, 1, 0);
   // A launch holds less than 2^32 threads (a larger one is not refused, its
   // workgroup count wraps): 2^24 workgroups and more on 2 wavefronts, too.
   const bool fits4 = (long)xcd_grid(batch, heads) * 256 < 1l << 32;
-  if (tiles >= (VL ? 4 : 2) && fits4) return BBH_ATT(4, 1, 3);
+  if (tiles >= (VL ? 4 : wgs > 1536 ? 3 : 2) && fits4) return BBH_ATT(4, 1, 3);
   if (tiles >= 2) return BBH_ATT(2, 1, 3);
   return BBH_ATT(1, 1, 3);
 #undef BBH_ATT

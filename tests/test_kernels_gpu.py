@@ -348,11 +348,13 @@ def test_attention_bits_do_not_depend_on_the_padding(torch_cuda):
             assert np.abs(got.astype(np.float32) - ref.astype(np.float32)).max() <= 4e-3, (n, S)
 
 
-@pytest.mark.parametrize("B,S", [(107, 288), (110, 352), (107, 368), (172, 496), (256, 512),
-                                 (60, 256), (300, 96)])
+@pytest.mark.parametrize("B,S", [(43, 288), (64, 320), (107, 288), (110, 352), (107, 368),
+                                 (172, 496), (256, 512), (60, 256), (300, 96), (128, 48), (129, 48),
+                                 (129, 64)])
 def test_attention_bits_do_not_depend_on_the_batch(torch_cuda, B, S):
     # From 1281 (sequence, head) pairs on, 9-11 query tiles run on 8 wavefronts
-    # instead of 12; 8 and 16 tiles take one shape in every batch (two tiles a
+    # instead of 12, 9 and 10 also at 513-768 and 1025-1280, two tiles on 2 instead
+    # of 4 from 1537 on; 8 and 16 tiles take one shape in every batch (two tiles a
     # wavefront).  The rows of a sentence are, bit for bit, those it has in a
     # batch of three, scores rising along the keys included, and close to fp32.
     # (256 x 512 also walks the sequences from the last one.)
