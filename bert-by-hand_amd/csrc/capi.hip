@@ -610,7 +610,7 @@ bbh_status run_layers_carried(bbh_workspace* ws, const bbh_model* m, f16* h0, co
     const bbh_model::Layer* P = i > 0 ? &m->layers[i - 1] : nullptr;  // its ln2 normalises cur
     const bool last = i == BBH_NUM_LAYERS - 1;
     f16* nxt = last ? final_out : (cur == ws->ping ? ws->pong : ws->ping);
-    const int qkv_tile = bbh::gemm_tile(M, 3 * H, H, sh);
+    const int qkv_tile = bbh::gemm_tile(M, 3 * H, H, sh, P != nullptr);
     if (fused_qa) {
       // QKV Linear and attention in one kernel (timing record: fused_ln 3)
       bbh::LnCarry cy;
@@ -663,7 +663,7 @@ bbh_status run_layers_carried(bbh_workspace* ws, const bbh_model* m, f16* h0, co
       cy.mr_out = ws->mr_a;
       cy.fs = L.f1_fs;
       cy.fc = L.f1_fc;
-      BBH_TRY(timed_op(t, s, {BBH_OP_FFN1_GELU, bbh::gemm_tile(M, F, H, sh), 2, M, F, H, 0.f}, [&] {
+      BBH_TRY(timed_op(t, s, {BBH_OP_FFN1_GELU, bbh::gemm_tile(M, F, H, sh, true), 2, M, F, H, 0.f}, [&] {
         return check_launch(bbh::gemm_fold(ws->attn_out, L.f1_wf, cy, ws->inter, M, F, H,
                                            bbh::Act::kGelu, eps, s, sh),
                             "ffn1 gemm (carried LayerNorm)");

@@ -1868,7 +1868,7 @@ int pick_deep(int M, int N, int K) {
   return -1;
 }
 
-int pick_plain(int M, int N, int K, bool shared) {
+int pick_plain(int M, int N, int K, bool shared, bool fold = false) {
   const bool qkv = N == 1152, ffn1 = N == 1536, wide_k = K >= 1024;
   int id = shared ? -1 : pick_deep(M, N, K);
   if (id >= 0) return id;
@@ -1883,7 +1883,7 @@ int pick_plain(int M, int N, int K, bool shared) {
   else if (M <= 6144)
     id = qkv ? 30 : ffn1 ? (shared ? 26 : 19) : wide_k ? 31 : 0;
   else if (M <= 8192)
-    id = shared ? (wide_k ? 31 : 30) : qkv || ffn1 ? 19 : wide_k ? 30 : 0;
+    id = shared ? (wide_k ? 31 : 30) : ffn1 || (qkv && (fold || M > 7168)) ? 19 : qkv || wide_k ? 30 : 0;
   else if (M <= 16384)
     id = !wide_k ? 30
          : M <= 10880 && N % 128 == 0 && (long)((M + 127) / 128) * (N / 128) > kCus * 5 / 4 ? 40
@@ -1899,9 +1899,9 @@ int pick_plain(int M, int N, int K, bool shared) {
 
 bool gemm_mfma_ok(int N, int K) { return N % 64 == 0 && K % 64 == 0; }
 
-int gemm_tile(int M, int N, int K, bool shared) {
+int gemm_tile(int M, int N, int K, bool shared, bool fold) {
   if (!gemm_mfma_ok(N, K)) return -1;
-  return wres_ok(M, N, K) ? kTiles : pick_plain(M, N, K, shared);
+  return wres_ok(M, N, K) ? kTiles : pick_plain(M, N, K, shared, fold);
 }
 
 // Large M: one kernel that owns whole rows.  Smaller M: a tile that owns whole
@@ -2096,7 +2096,7 @@ hipError_t gemm_fold(const f16* A, const f16* W, const LnCarry& cy, f16* C, int 
   if (!ln_carry_ok(M) || !gemm_mfma_ok(N, K) || !aligned || !cy.st_in || !cy.fs || !cy.fc ||
       wres_ok(M, N, K))
     return hipErrorInvalidValue;
-  const int id = pick_plain(M, N, K, shared);
+  const int id = pick_plain(M, N, K, shared, true);
   return act == Act::kGelu
              ? launch_carry<kFoldGelu>(id, A, W, nullptr, nullptr, nullptr, nullptr, C, M, N, K, eps, s, cy)
              : launch_carry<kFold>(id, A, W, nullptr, nullptr, nullptr, nullptr, C, M, N, K, eps, s, cy);

@@ -69,10 +69,10 @@ hipError_t qkv_attention(const f16* X, const f16* Wp, const float* fs, const flo
                          const LnCarry& cy, const int32_t* mask, f16* ctx, int batch, int seq,
                          float scale, float eps, hipStream_t s, bool shared = false);
 
-// Tile configuration gemm() / gemm_residual_ln() launch for a shape (-1: the
-// plain tiled kernel), whether the LayerNorm is inside the GEMM kernel, and
-// the configuration's name as it appears in the kernel symbol.
-int gemm_tile(int M, int N, int K, bool shared = false);
+// Tile configuration gemm(), gemm_fold() (fold) or gemm_residual_ln() launch for
+// a shape (-1: the plain tiled kernel), whether the LayerNorm is inside the GEMM
+// kernel, and the configuration's name as it appears in the kernel symbol.
+int gemm_tile(int M, int N, int K, bool shared = false, bool fold = false);
 int gemm_residual_ln_tile(int M, int K, bool* fused_ln, bool shared = false, bool sliced = false);
 const char* gemm_tile_name(int tile);
 // Work-items of a launch of a tile (0: not a tile of the table), and the

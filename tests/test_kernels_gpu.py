@@ -449,7 +449,9 @@ def test_residual_layernorm_rows_above_8192(torch_cuda, K):
     (384, 1088, (16, 2500)), (64, 1024, (8000,)),
     # K < 1024: 32x64, 64x64, 96x64, 64x128; three slices, one slice.
     (384, 384, (16, 1345, 2689, 4033, 5440)), (1536, 384, (320, 321, 641, 961, 1344, 1345)),
-    (1152, 192, (31, 449)), (128, 64, (1, 4097))])
+    (1152, 192, (31, 449)), (128, 64, (1, 4097)),
+    # N = 1152 past one round of 128x128 tiles
+    (1152, 384, (7168, 7169))])
 def test_linear_rows_do_not_depend_on_the_tile(torch_cuda, N, K, Ms):
     # Every tile adds k in the same order and rounds the same way: the rows of
     # any row count are, bit for bit, those of a call with 50000 rows.
