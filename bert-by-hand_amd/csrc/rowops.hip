@@ -319,14 +319,12 @@ __global__ __launch_bounds__(256) void mean_pool_kernel(const f16* __restrict__ 
   out[idx] = (f16)(acc / (float)(cnt > 0 ? cnt : 1));
 }
 
-// The same for dim % 8 == 0 up to kPoolThreads columns of eight and batches
-// below 2^22 (a launch holds less than 2^32 threads; a larger one is not
-// refused, its workgroup count wraps): one workgroup per sentence, eight
-// columns a thread, the positions dealt to as many row groups as the threads
-// allow and the groups' sums added through LDS.  Masked rows are not read.
-// Bound by the row loads' latency, four of which a thread keeps in flight: 128 x
-// 112 rows of 384 took 50.6 us with one thread a column walking the mask,
-// against 6.1 us here.
+// The same for dim % 8 == 0 up to kPoolThreads columns of eight: one workgroup
+// per sentence, eight columns a thread, the positions dealt to as many row
+// groups as the threads allow and the groups' sums added through LDS.  Masked
+// rows are not read.  Bound by the row loads' latency, four of which a thread
+// keeps in flight: 128 x 112 rows of 384 took 50.6 us with one thread a column
+// walking the mask, against 6.1 us here.
 constexpr int kPoolThreads = 1024;
 __global__ __launch_bounds__(kPoolThreads) void mean_pool8_kernel(
     const f16* __restrict__ hidden, const int32_t* __restrict__ mask, f16* __restrict__ out,
@@ -468,9 +466,29 @@ hipError_t embedding_ln(const int32_t* ids, const int32_t* types, const f16* wor
   return hipGetLastError();
 }
 
+// Where a workgroup a sentence pays (sentences x seq x dim, us, one thread a
+// column -> here):
+//  - from kPoolSeq positions, else there is no walk to share (256 x 4 x 384 2.9 ->
+//    3.2, 256 x 16 x 384 5.3 -> 3.8);
+//  - with most of its threads at work, or all workgroups resident, two a CU
+//    (2000 x 16 x 64 5.4 -> 8.0, 20000 x 16 x 64 32 -> 73; 256 x 16 x 64 4.9 -> 3.1, 2000 x
+//    16 x 384 17.3 -> 13.1);
+//  - up to 1024 columns, or with a sentence for every CU, else fewer CUs work
+//    than with a thread a column (16 x 16 x 4096 4.8 -> 5.3, 1 x 512 x 8192 93 -> 180;
+//    256 x 16 x 4096 21 -> 6.7);
+//  - below 2^22 sentences: a launch holds less than 2^32 threads (a larger one is
+//    not refused, its workgroup count wraps).
+constexpr int kPoolSeq = 8;
+bool pool8_pays(int batch, int seq, int dim) {
+  if (dim % 8 != 0 || dim / 8 > kPoolThreads || batch >= (1ll << 32) / kPoolThreads) return false;
+  const int cols = dim / 8, busy = cols * std::min(kPoolThreads / cols, seq);
+  return seq >= kPoolSeq && (busy >= kPoolThreads * 3 / 4 || batch <= 512) &&
+         (dim <= 1024 || batch >= 256);
+}
+
 hipError_t mean_pool(const f16* hidden, const int32_t* mask, f16* out, int batch, int seq,
                      int dim, hipStream_t s) {
-  if (dim % 8 == 0 && dim / 8 <= kPoolThreads && batch < (1ll << 32) / kPoolThreads) {
+  if (pool8_pays(batch, seq, dim)) {
     const int groups = std::min(kPoolThreads / (dim / 8), seq);
     const size_t lds = (size_t)groups * (dim + 1) * sizeof(float);  // at most 36 KB
     hipLaunchKernelGGL(mean_pool8_kernel, dim3(batch), dim3(kPoolThreads), lds, s, hidden, mask,

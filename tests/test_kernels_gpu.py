@@ -517,10 +517,14 @@ def test_unfused_attention_pieces_edges(torch_cuda, B, S, off):
 
 
 @pytest.mark.parametrize("B,S,D,off", [(1, 1, 8, 0), (3, 7, 384, 1), (2, 512, 384, 0), (2, 40, 1032, 0),
-                                       (5, 33, 100, 0), (1, 90, 8200, 0), (2, 3, 512, 1)])
+                                       (5, 33, 100, 0), (1, 90, 8200, 0), (2, 3, 512, 1),
+                                       # the pool's workgroup a sentence, at its edges
+                                       (2, 8, 8, 0), (3, 9, 384, 1), (2, 40, 1024, 0), (600, 12, 512, 1),
+                                       (600, 8, 384, 0), (256, 8, 8192, 0)])
 def test_row_operators_edges(torch_cuda, B, S, D, off):
     # embedding, mean pool and L2 normalise at any width (the vector kernels
-    # take D % 8 == 0, up to 8192 and 512 columns), at odd element addresses,
+    # take D % 8 == 0, the pool's up to 8192 columns where it pays, the
+    # normalise's up to 512), at odd element addresses,
     # with an all-masked sentence; NaN in masked rows is not read.  Bounds as
     # above; the embedding is exact up to its fp16 rounding.
     torch = torch_cuda
