@@ -1843,7 +1843,7 @@ const char* tile_name(int id) {
 // GEMM is bound by one workgroup's walk over K, which a smaller tile
 // shortens (fewer bytes through its CU per slice); one workgroup more than
 // CUs would start a second round.  Against the tiles that ran before, back to
-// back launches on one box: FFN2 at 16 / 1024 / 2048 / 3072 / 4096 / 6144 /
+// back launches on one GPU: FFN2 at 16 / 1024 / 2048 / 3072 / 4096 / 6144 /
 // 8192 rows 9.6 / 10.3 / 10.5 / 11.4 / 12.0 / 16.1 / 17.6 -> 5.7 / 6.1 / 7.1 /
 // 8.6 / 10.0 / 12.4 / 15.6 us; O-proj at 16 / 1024 / 2048 / 3072 / 4096 rows
 // 4.0 / 4.4 / 4.5 / 4.9 / 5.1 -> 2.9 / 3.2 / 3.7 / 4.5 / 4.8; FFN1 at 16 /
