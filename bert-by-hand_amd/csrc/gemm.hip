@@ -1813,7 +1813,11 @@ const char* tile_name(int id) {
 // past them, from sweeps with one GEMM's tile changed at a time:
 //  - QKV: the 64x64 copy-ring tile (0) up to 2048 rows (inside bert_embed 4 x 512
 //    304 us against 307 on tile 30, and below, on pick_deep's tiles, 6 x 256 227
-//    against 235; back to back the two are level at 1700-2048 rows).
+//    against 235; back to back the two are level at 1700-2048 rows).  At 6145-8192
+//    rows 256x192 (19) with a carried LayerNorm coming in (fold: bert_embed 43 x
+//    144 / 50 x 144 404 / 430 us against 411 / 454 on tile 30); without it tile 30 up
+//    to 7168 rows, one round of two workgroups a CU (6500 / 7000 rows 11.1 / 11.6 us
+//    against 13.1 / 13.2 on 19; 7300 rows 14.4 against 13.5).
 //  - FFN1: tile 0 to 4096 rows (one-slot pass 8.22-8.24 -> 8.11 ms against the
 //    register-staged 64x64 at 2049-3072 rows): more workgroups than CUs keep
 //    every CU busy.  At 4097-8192 rows 256x192 (19), which covers 8192 rows with
@@ -1834,9 +1838,10 @@ const char* tile_name(int id) {
 // tiles 36-39 cost 2.7 to 5.5% there.  The other forwards fill the CUs, and
 // fewer, larger tiles move fewer bytes L2 -> CU per FLOP.
 // A forward on one of several streams that a caller drives without a pool counts
-// as alone: four of 64 x 32 on four streams take 107 us each against 102 with the
-// tiles of the pool, two on two 119 against 128; 64 x 16 64 against 73, 64 x 64 181
-// against 195, 64 x 128 339 against 345 on four.
+// as alone.  Against smaller rings (tiles 0, 26, 30 and 128-row QKV + attention),
+// four of 64 x 32 on four streams take 107 us each instead of 102, but two on two
+// 119 instead of 128, and on four 64 x 16 64 instead of 73, 64 x 64 181 instead of
+// 195, 64 x 128 339 instead of 345.
 //
 // Alone, where one workgroup per CU covers the output (kCus CUs): the smallest
 // of the mainloop_deep tiles that needs at most kCus workgroups.  Such a
